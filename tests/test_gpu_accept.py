@@ -218,3 +218,48 @@ def test_truncation_tie_group_spanning_late_id_steps(dev, stream):
     for top_k, top_p in [(120, 1.0), (0, 0.5), (250, 0.3), (41, 1.0)]:
         for step in range(2):
             assert _check_truncated(dev, stream, logits, drafts, 1.0, top_k, top_p, 21, step) == 0
+
+
+# Rows up to 8192 logits are cut in LDS whole; longer ones through the binned
+# candidates: by counting up to 512, by radix selection above, over the whole
+# row where the candidates do not fit (a sorted row fills one wave's segment,
+# equal logits one bin, a masked row ends in the open last bin).
+@pytest.mark.parametrize("V,shape,top_k,top_p,T", [
+    (8192, "normal", 0, 0.9, 0.7), (8193, "normal", 0, 0.9, 0.7), (8193, "normal", 513, 0.97, 1.0),
+    (40001, "narrow", 0, 0.6, 1.0), (40001, "normal", 511, 1.0, 0.8), (40001, "normal", 6000, 0.999, 1.3),
+    (40001, "sorted", 200, 0.95, 1.0), (40001, "sorted", 0, 0.95, 1.0), (20000, "equal", 0, 0.5, 1.0),
+    (20000, "equal", 300, 0.5, 1.0), (40001, "masked", 40, 0.9, 0.7), (40001, "masked", 0, 0.999, 1.0),
+    (40001, "outlier", 0, 0.9, 1.0), (300, "normal", 20, 0.9, 0.7)])
+def test_truncation_paths_match_oracle(dev, stream, V, shape, top_k, top_p, T):
+    rng = np.random.default_rng(V + top_k)
+    k = 3
+    logits = rng.normal(0, {"narrow": 1e-3}.get(shape, 3), (k + 1, V)).astype(np.float32)
+    if shape == "sorted":
+        logits = -np.sort(-logits, axis=1)
+    if shape == "equal":
+        logits[:] = 0.25
+    if shape == "masked":
+        logits[rng.random(logits.shape) < 0.98] = -np.inf
+    if shape == "outlier":
+        logits[:, V // 2] = -1e30
+    drafts = np.argsort(-logits, axis=1, kind="stable")[np.arange(k), [0, 1, 5]].astype(np.int32)
+    for step in range(3):
+        assert _check_truncated(dev, stream, logits, drafts, T, top_k, top_p, 19, step) == 0
+
+
+@pytest.mark.parametrize("B", [2, 160, 400, 900])
+def test_truncated_batch_equals_requests_alone(dev, stream, B):
+    """More rows leave fewer bins and candidates per row; the kept sets and
+    the decisions are those of each request alone."""
+    rng = np.random.default_rng(B)
+    k, V = 2, 9001
+    logits = rng.normal(0, 3, (B, k + 1, V)).astype(np.float32)
+    drafts = logits[:, :k].argmax(2).astype(np.int32)
+    for top_k, top_p in [(0, 0.9), (50, 0.8)]:
+        p = hip.accept_params(hip.ACCEPT_STOCHASTIC, B, k, V, temperature=0.9, top_k=top_k, top_p=top_p, seed=5)
+        res, _ = _run(dev, stream, logits, drafts, p)
+        for b in (0, B // 2, B - 1):
+            one = hip.accept_params(hip.ACCEPT_STOCHASTIC, 1, k, V, temperature=0.9, top_k=top_k, top_p=top_p, seed=5,
+                                    request_base=b)
+            alone, _ = _run(dev, stream, logits[b], drafts[b], one)
+            assert res[b].tolist() == alone[0].tolist(), b

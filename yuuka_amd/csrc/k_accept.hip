@@ -11,17 +11,29 @@
 //
 // Kernels (the passes over a row are separate launches so that the exact row
 // maximum is known before any exponential is taken):
-//   1. stats:    per (request, row, chunk): maximum and its first index.
-//   2. select:   (top-k / top-p only) one workgroup per row finds the row's
-//                cut by radix selection over the order key of the logits.
-//   3. weights:  (stochastic) per chunk: float64 sum of the kept weights with
-//                the draft removed, and the draft's own weight.
-//   4. finalize: one workgroup per request walks the rows in order, decides,
-//                and for a rejection or the bonus row draws by inverse CDF
-//                in index order (chunk prefix, then a scan inside the chunk).
+//   stats:    per (request, row, chunk): maximum and its first index.
+// greedy and untruncated stochastic:
+//   weights:  (stochastic) per chunk: float64 sum of the weights with the
+//             draft removed, and the draft's own weight.
+//   finalize: one workgroup per request walks the rows in order, decides,
+//             and for a rejection or the bonus row draws by inverse CDF
+//             in index order (chunk prefix, then a scan inside the chunk).
+// top-k / top-p:
+//   bins:     per (row, chunk) histogram of the row over equal steps of the
+//             logit below the row maximum.
+//   collect:  the bin that holds the cut, and its members (top-k: every
+//             member down to it) as a candidate list.
+//   cut:      one workgroup per row finds the exact cut among the candidates
+//             (or over the whole row when they do not fit), and the weight
+//             sums of the kept set.
+//   resample: decides every request, and sums the kept weights of the one
+//             row it draws from, per chunk.
+//   pick:     the draw, as finalize makes it.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
+#include <type_traits>
 
 #include "internal.h"
 
@@ -48,30 +60,53 @@ __device__ __forceinline__ const float *row_ptr(const float *logits, const Geo &
     return logits + ((uint64_t)b * g.R + row) * g.stride;
 }
 
-// Per (request, row, chunk) maximum. A chunk of L (a multiple of 4) logits
-// is read by `wpc` waves (1: four chunks per workgroup, for short chunks;
-// 4: one chunk per workgroup), with 16-byte loads when the rows are 16-byte
-// aligned. The maximum under `beats` does not depend on the order in which
-// elements are visited, so the split does not change the result.
+// Bytes of truncation scratch per (request, row, chunk), and the sums of a
+// chunk's logits (up to 1e6 in size) that set the truncation's bin width.
+constexpr uint64_t kRowArea = 3072;
+struct Moments {
+    float n, s1, s2, pad;
+};
+
+__device__ __forceinline__ uint8_t *row_area(uint8_t *area, const Geo &g, int b, int row) {
+    return area + ((uint64_t)b * g.R + row) * g.C * kRowArea;
+}
+
+// Per (request, row, chunk) maximum (MOM: and the moments, at the start of
+// the row's area). A chunk of L (a multiple of 4) logits is read by `wpc`
+// waves (1: four chunks per workgroup, for short chunks; 4: one chunk per
+// workgroup), with 16-byte loads when the rows are 16-byte aligned. The
+// maximum under `beats` does not depend on the order in which elements are
+// visited, so the split does not change the result.
+template <bool MOM>
 __global__ __launch_bounds__(256) void accept_stats_kernel(const float *__restrict__ logits, Geo g,
-                                                           Stat *__restrict__ stats, int vec, int wpc) {
+                                                           Stat *__restrict__ stats, int vec, int wpc,
+                                                           uint8_t *__restrict__ area) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int c = blockIdx.x * (4 / wpc) + wave / wpc, row = blockIdx.y, b = blockIdx.z;
     const int t = (wave % wpc) * 64 + lane, nt = wpc * 64;
     const bool live = c < g.C;
     float bv = -INFINITY;
     int bi = INT_MAX;
+    float mn = 0.f, m1 = 0.f, m2 = 0.f;
+    auto take = [&](float v, int j) __attribute__((always_inline)) {
+        if (beats(v, j, bv, bi)) { bv = v; bi = j; }
+        if (MOM && fabsf(v) <= 1e6f) {
+            mn += 1.f;
+            m1 += v;
+            m2 = fmaf(v, v, m2);
+        }
+    };
     if (live) {
         const float *p = row_ptr(logits, g, b, row);
         const int begin = c * g.L;
         const int end = min(begin + g.L, g.V);
         if (vec) {
             const int end4 = begin + ((end - begin) & ~3);
-            auto take4 = [&](const float4 v, int j) {
-                if (beats(v.x, j, bv, bi)) { bv = v.x; bi = j; }
-                if (beats(v.y, j + 1, bv, bi)) { bv = v.y; bi = j + 1; }
-                if (beats(v.z, j + 2, bv, bi)) { bv = v.z; bi = j + 2; }
-                if (beats(v.w, j + 3, bv, bi)) { bv = v.w; bi = j + 3; }
+            auto take4 = [&](const float4 v, int j) __attribute__((always_inline)) {
+                take(v.x, j);
+                take(v.y, j + 1);
+                take(v.z, j + 2);
+                take(v.w, j + 3);
             };
             int j = begin + t * 4;
             // four 16-byte loads in flight per thread
@@ -84,18 +119,9 @@ __global__ __launch_bounds__(256) void accept_stats_kernel(const float *__restri
             }
             for (; j < end4; j += nt * 4) take4(*reinterpret_cast<const float4 *>(p + j), j);
             const int jt = end4 + t;
-            if (jt < end && beats(p[jt], jt, bv, bi)) {
-                bv = p[jt];
-                bi = jt;
-            }
+            if (jt < end) take(p[jt], jt);
         } else {
-            for (int j = begin + t; j < end; j += nt) {
-                const float v = p[j];
-                if (beats(v, j, bv, bi)) {
-                    bv = v;
-                    bi = j;
-                }
-            }
+            for (int j = begin + t; j < end; j += nt) take(p[j], j);
         }
     }
     for (int off = 32; off > 0; off >>= 1) {
@@ -105,19 +131,38 @@ __global__ __launch_bounds__(256) void accept_stats_kernel(const float *__restri
             bv = ov;
             bi = oi;
         }
+        if (MOM) {
+            mn += __shfl_xor(mn, off);
+            m1 += __shfl_xor(m1, off);
+            m2 += __shfl_xor(m2, off);
+        }
     }
+    Moments *mom = MOM && live ? reinterpret_cast<Moments *>(row_area(area, g, b, row)) + c : nullptr;
     if (wpc == 1) {
-        if (live && lane == 0) stats[((uint64_t)b * g.R + row) * g.C + c] = Stat{bv, bi};
+        if (live && lane == 0) {
+            stats[((uint64_t)b * g.R + row) * g.C + c] = Stat{bv, bi};
+            if (MOM) *mom = Moments{mn, m1, m2, 0.f};
+        }
         return;
     }
     __shared__ Stat ws[4];
-    if (lane == 0) ws[wave] = Stat{bv, bi};
+    __shared__ Moments wm[4];
+    if (lane == 0) {
+        ws[wave] = Stat{bv, bi};
+        wm[wave] = Moments{mn, m1, m2, 0.f};
+    }
     __syncthreads();
     if (threadIdx.x == 0 && live) {
         Stat s = ws[0];
-        for (int w = 1; w < 4; w++)
+        Moments m = wm[0];
+        for (int w = 1; w < 4; w++) {
             if (beats(ws[w].v, ws[w].i, s.v, s.i)) s = ws[w];
+            m.n += wm[w].n;
+            m.s1 += wm[w].s1;
+            m.s2 += wm[w].s2;
+        }
         stats[((uint64_t)b * g.R + row) * g.C + c] = s;
+        if (MOM) *mom = m;
     }
 }
 
@@ -148,45 +193,123 @@ __device__ __forceinline__ bool in_cut(uint32_t key, int j, const Cut &c) {
     return key > c.key || (key == c.key && j <= c.id);
 }
 
-// exp(float64(logit - max) / T) (sampling.go:97), zero outside the cut.
-__device__ __forceinline__ double weight_of(float l, int j, float mx, double t, const Cut &c) {
-    if (!valid_logit(l) || !in_cut(order_key(l), j, c)) return 0.0;
-    return exp((double)(l - mx) / t);
+// The temperature as the weights use it: 1 / t rounded, and t for the
+// residual that makes the quotient below correctly rounded (up to its last
+// few denormals).
+struct Temp {
+    double t, rt;
+};
+
+// (logit - max) / T; -inf stays out of the residual.
+__device__ __forceinline__ double exponent_of(float l, float mx, const Temp &t) {
+    float d = l - mx;
+    d = d == -INFINITY ? -3.4e38f : d;
+    const double a = (double)d, q = a * t.rt;
+    return fma(fma(-q, t.t, a), t.rt, q);
 }
 
-__device__ __forceinline__ Cut row_cut(const Cut *cuts, const Geo &g, int b, int row) {
-    return cuts ? cuts[(uint64_t)b * g.R + row] : Cut{0u, INT_MAX};
+// exp(x) for x <= 0 (NaN stays NaN): 2^k e^r with r = x - k ln 2 in two FMA
+// steps (|r| <= 0.35) and the Taylor series of e^r to r^13 (its remainder is
+// below 5e-18).
+__device__ __forceinline__ double exp_nonpos(double x) {
+    const double k = rint(x * 0x1.71547652b82fep+0);
+    const double r = fma(k, -0x1.abc9e3b39803fp-56, fma(k, -0x1.62e42fefa39efp-1, x));
+    double p = 1.0 / 6227020800.0;
+    p = fma(p, r, 1.0 / 479001600.0);
+    p = fma(p, r, 1.0 / 39916800.0);
+    p = fma(p, r, 1.0 / 3628800.0);
+    p = fma(p, r, 1.0 / 362880.0);
+    p = fma(p, r, 1.0 / 40320.0);
+    p = fma(p, r, 1.0 / 5040.0);
+    p = fma(p, r, 1.0 / 720.0);
+    p = fma(p, r, 1.0 / 120.0);
+    p = fma(p, r, 1.0 / 24.0);
+    p = fma(p, r, 1.0 / 6.0);
+    p = fma(p, r, 0.5);
+    p = fma(p, r, 1.0);
+    p = fma(p, r, 1.0);
+    const double e = ldexp(p, (int)k);
+    return x < -760.0 ? 0.0 : e;  // below the smallest denormal (k may be anything there)
+}
+
+// exp(x) for x <= 0 for the pass that weighs a whole vocabulary, which its
+// float64 operations bound: 2^(k/16) (and its rounding error) from a table
+// in LDS, e^r for |r| <= ln 2 / 32 to r^7 (remainder below 2e-18). Within
+// 0.6 ulp; with the plain series the pass took 51 us at 144 rows of 151936.
+__constant__ double2 kExpTab[16] = {
+    {0x1.0000000000000p+0, 0x0.0p+0}, {0x1.0b5586cf9890fp+0, 0x1.8a62e4adc610bp-54},
+    {0x1.172b83c7d517bp+0, -0x1.19041b9d78a76p-55}, {0x1.2387a6e756238p+0, 0x1.9b07eb6c70573p-54},
+    {0x1.306fe0a31b715p+0, 0x1.6f46ad23182e4p-55}, {0x1.3dea64c123422p+0, 0x1.ada0911f09ebcp-55},
+    {0x1.4bfdad5362a27p+0, 0x1.d4397afec42e2p-56}, {0x1.5ab07dd485429p+0, 0x1.6324c054647adp-54},
+    {0x1.6a09e667f3bcdp+0, -0x1.bdd3413b26456p-54}, {0x1.7a11473eb0187p+0, -0x1.41577ee04992fp-55},
+    {0x1.8ace5422aa0dbp+0, 0x1.6e9f156864b27p-54}, {0x1.9c49182a3f090p+0, 0x1.c7c46b071f2bep-56},
+    {0x1.ae89f995ad3adp+0, 0x1.7a1cd345dcc81p-54}, {0x1.c199bdd85529cp+0, 0x1.11065895048ddp-55},
+    {0x1.d5818dcfba487p+0, 0x1.2ed02d75b3707p-55}, {0x1.ea4afa2a490dap+0, -0x1.e9c23179c2893p-54}};
+__device__ __forceinline__ double exp_nonpos_tab(double x, const double2 *tab) {
+    const double k = rint(x * 0x1.71547652b82fep+4);
+    const double r = fma(k, -0x1.abc9e3b39803fp-60, fma(k, -0x1.62e42fefa39efp-5, x));
+    double p = fma(r, 1.0 / 5040.0, 1.0 / 720.0);
+    p = fma(p, r, 1.0 / 120.0);
+    p = fma(p, r, 1.0 / 24.0);
+    p = fma(p, r, 1.0 / 6.0);
+    p = fma(p, r, 0.5);
+    p = fma(p, r, 1.0);
+    const int ki = (int)k;
+    const double2 f = tab[ki & 15];
+    const double e = ldexp(f.x + fma(f.x, p * r, f.y), ki >> 4);
+    return x < -760.0 ? 0.0 : e;
+}
+
+// exp(float64(logit - max) / T) (sampling.go:97) of a valid logit.
+__device__ __forceinline__ double soft_weight(float l, float mx, const Temp &t) {
+    return exp_nonpos(exponent_of(l, mx, t));
+}
+
+// The same, zero outside the cut.
+__device__ __forceinline__ double weight_of(float l, int j, float mx, const Temp &t, const Cut &c) {
+    if (!valid_logit(l) || !in_cut(order_key(l), j, c)) return 0.0;
+    return soft_weight(l, mx, t);
+}
+
+// Wave 0 of a workgroup: the row's maximum and its first index over the
+// chunk statistics, in every lane.
+__device__ __forceinline__ Stat wave_best(const Stat *__restrict__ st, int C) {
+    const int lane = threadIdx.x & 63;
+    Stat s{-INFINITY, INT_MAX};
+    for (int cc = lane; cc < C; cc += 64)
+        if (beats(st[cc].v, st[cc].i, s.v, s.i)) s = st[cc];
+    for (int off = 32; off > 0; off >>= 1) {
+        const float ov = __shfl_xor(s.v, off);
+        const int oi = __shfl_xor(s.i, off);
+        if (beats(ov, oi, s.v, s.i)) s = Stat{ov, oi};
+    }
+    return s;
 }
 
 __global__ __launch_bounds__(256) void accept_weights_kernel(const float *__restrict__ logits, Geo g,
                                                              const int32_t *__restrict__ drafts,
-                                                             const Stat *__restrict__ stats,
-                                                             const Cut *__restrict__ cuts, double t,
+                                                             const Stat *__restrict__ stats, Temp t,
                                                              double *__restrict__ sums,
                                                              double *__restrict__ wdraft) {
     const int c = blockIdx.x, row = blockIdx.y, b = blockIdx.z;
     const float *p = row_ptr(logits, g, b, row);
     __shared__ float mx_s;
-    if (threadIdx.x < 64) {  // wave 0 reduces the row's chunk maxima
-        const Stat *st = stats + ((uint64_t)b * g.R + row) * g.C;
-        float bv = -INFINITY;
-        int bi = INT_MAX;
-        for (int cc = threadIdx.x; cc < g.C; cc += 64)
-            if (beats(st[cc].v, st[cc].i, bv, bi)) { bv = st[cc].v; bi = st[cc].i; }
-        for (int off = 32; off > 0; off >>= 1) {
-            const float ov = __shfl_xor(bv, off);
-            const int oi = __shfl_xor(bi, off);
-            if (beats(ov, oi, bv, bi)) { bv = ov; bi = oi; }
-        }
-        if (threadIdx.x == 0) mx_s = bv;
+    __shared__ double2 tab[16];
+    if (threadIdx.x < 16) tab[threadIdx.x] = kExpTab[threadIdx.x];
+    if (threadIdx.x < 64) {
+        const Stat s = wave_best(stats + ((uint64_t)b * g.R + row) * g.C, g.C);
+        if (threadIdx.x == 0) mx_s = s.v;
     }
     __syncthreads();
     const float mx = mx_s;
-    const Cut cut = row_cut(cuts, g, b, row);
     const int d = row < g.k ? drafts[(uint64_t)b * g.ds + row] : -1;
     const int begin = c * g.L;
     const int end = min(begin + g.L, g.V);
     double acc = 0.0;
+    auto weigh = [&](float l) __attribute__((always_inline)) {
+        const double w = exp_nonpos_tab(exponent_of(l, mx, t), tab);
+        return valid_logit(l) ? w : 0.0;
+    };
     // eight logit loads in flight per thread; the sum keeps index order
     constexpr int kU = 8;
     int j = begin + threadIdx.x;
@@ -194,9 +317,12 @@ __global__ __launch_bounds__(256) void accept_weights_kernel(const float *__rest
         float l[kU];
 #pragma unroll
         for (int u = 0; u < kU; u++) l[u] = p[j + u * 256];
+        double wv[kU];
+#pragma unroll
+        for (int u = 0; u < kU; u++) wv[u] = weigh(l[u]);
 #pragma unroll
         for (int u = 0; u < kU; u++) {
-            const double w = weight_of(l[u], j + u * 256, mx, t, cut);
+            const double w = wv[u];
             if (j + u * 256 == d)
                 wdraft[(uint64_t)b * g.R + row] = w;
             else
@@ -204,7 +330,7 @@ __global__ __launch_bounds__(256) void accept_weights_kernel(const float *__rest
         }
     }
     for (; j < end; j += 256) {
-        const double w = weight_of(p[j], j, mx, t, cut);
+        const double w = weigh(p[j]);
         if (j == d)
             wdraft[(uint64_t)b * g.R + row] = w;
         else
@@ -218,10 +344,313 @@ __global__ __launch_bounds__(256) void accept_weights_kernel(const float *__rest
 }
 
 // ---------------------------------------------------------------- truncation
-// Per-row cut for top-k / top-p (sampling.go:84-113) without sorting: radix
-// selection over the 32-bit order key, one workgroup per row, histograms in
-// LDS. Each wave fills its own histogram and the waves are combined in wave
-// order, so weight sums do not depend on wave scheduling.
+// Per-row cut for top-k / top-p (sampling.go:84-113) without sorting.
+//
+// A histogram over equal steps of the logit below the row maximum, one
+// workgroup per (row, chunk), leaves a few hundred candidates around the cut
+// for any smooth distribution; one workgroup per row then orders those
+// exactly. (A histogram over the top byte of the order key, as a radix
+// selection has it, has about five buckets in use at once — an octave or two
+// each — so the 64 lanes of an LDS atomic met on the same few addresses
+// (95 us at 144 rows of 151936), and its boundary bucket still held 17
+// thousand members, for three more passes of one workgroup per row (136 us).)
+// Rows whose candidates do not fit (a bin of many equal logits, or a cut in
+// the open last bin) take the radix selection over the whole row.
+//
+// Scratch of one (request, row): C * kRowArea bytes of
+//   Moments [C]              per-chunk sums behind the bin width
+//   double or uint32 [HC][NB]  chunk histograms: weights, or counts with top-k
+//   uint32 [segs]            candidates of each collecting wave
+//   Member [segs][seg]       the candidates
+constexpr int kBins = 1024;    // most bins of a histogram
+constexpr int kBinWaves = 8;   // waves of a bins workgroup, a histogram each
+constexpr int kCandMost = 8192;
+constexpr int kDirectMost = 8192;  // vocabulary whose rows go to LDS whole
+constexpr int kRankMost = 512;  // candidates ordered by counting
+
+struct Member {
+    float l;
+    int j;
+};
+
+struct TruncGeo {
+    int NB;    // bins
+    int HC;    // histogram chunks of a row
+    int KC;    // collecting chunks of a row (4 waves each)
+    int seg;   // candidates of one collecting wave
+    uint32_t bins_off, cnt_off, cand_off;  // in the row's area
+};
+
+// What collect leaves for a row.
+struct RowCut {
+    Cut cut;
+    double rest;   // kept weight without the draft
+    double wd;     // the draft's kept weight
+    double total;  // (collect -> cut) all weight, draft included
+    double before;       // (collect -> cut) weight above the boundary bin, draft included
+    double before_rest;  // ... without the draft
+    float best_v;        // row maximum
+    int best_i;
+    int status;  // kCutFound: the candidates decide; kCutAll: nothing is cut; kCutRow: scan the row
+    int pad;
+};
+enum { kCutFound = 0, kCutAll = 1, kCutRow = 2 };
+
+// A row's record lies at the end of its area.
+__device__ __forceinline__ RowCut &row_cut(uint8_t *area, const Geo &g, int b, int row) {
+    return *reinterpret_cast<RowCut *>(row_area(area, g, b, row) + g.C * kRowArea - sizeof(RowCut));
+}
+
+// Bins per unit of logit below the maximum: the range down to three standard
+// deviations under the mean, or 48 T if that is less (the weights below it
+// are under 1e-20 of the largest), in NB steps. Every workgroup of a row
+// computes the same value (fixed order), so the bins of its passes agree.
+// Wave 0 of a workgroup.
+__device__ __forceinline__ float wave_bin_scale(const Moments *__restrict__ m, int C, float mx, const Temp &t, int NB) {
+    const int lane = threadIdx.x & 63;
+    float n = 0.f, s1 = 0.f, s2 = 0.f;
+    for (int c = lane; c < C; c += 64) {
+        n += m[c].n;
+        s1 += m[c].s1;
+        s2 += m[c].s2;
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        n += __shfl_xor(n, off);
+        s1 += __shfl_xor(s1, off);
+        s2 += __shfl_xor(s2, off);
+    }
+    const float cap = fminf(fmaxf(48.f * (float)t.t, 1e-30f), 1e30f);
+    const float mean = s1 / n;
+    const float sd = sqrtf(fmaxf(s2 / n - mean * mean, 1e-6f * mean * mean));
+    float range = (mx - mean) + 3.f * sd;
+    if (!(range > 1e-30f && range < cap)) range = cap;
+    return (float)NB / range;
+}
+
+// Monotone: a larger logit never has a larger bin (each operation rounds
+// monotonically; the last bin is open, and takes a NaN).
+__device__ __forceinline__ int bin_of(float l, float mx, float scale, int NB) {
+    return (int)fminf((mx - l) * scale, (float)(NB - 1));
+}
+
+// Histogram of one chunk of a row, the draft's weight left out. COUNT (with
+// top-k): members; otherwise their float64 weights. Each wave has its own
+// histogram (an atomic's lanes add in a fixed order, waves would not), the
+// waves are added in wave order.
+template <bool COUNT>
+__global__ __launch_bounds__(64 * kBinWaves) void accept_bins_kernel(const float *__restrict__ logits, Geo g, TruncGeo tg,
+                                                                     const int32_t *__restrict__ drafts,
+                                                                     const Stat *__restrict__ stats, Temp t,
+                                                                     uint8_t *__restrict__ area) {
+    using T = typename std::conditional<COUNT, uint32_t, double>::type;
+    extern __shared__ __attribute__((aligned(16))) uint8_t bins_dyn[];
+    T *hist = reinterpret_cast<T *>(bins_dyn);  // [wave][NB]
+    __shared__ float mx_s, scale_s;
+    __shared__ double2 tab[16];
+    if (!COUNT && threadIdx.x < 16) tab[threadIdx.x] = kExpTab[threadIdx.x];
+    constexpr int kT = 64 * kBinWaves;
+    const int c = blockIdx.x, row = blockIdx.y, b = blockIdx.z;
+    const float *p = row_ptr(logits, g, b, row);
+    uint8_t *ra = row_area(area, g, b, row);
+    const int begin = (int)((int64_t)g.V * c / tg.HC), end = (int)((int64_t)g.V * (c + 1) / tg.HC);
+    constexpr int kU = 8;  // loads in flight per thread
+    float lv[kU];
+    int j0 = begin + threadIdx.x;
+#pragma unroll
+    for (int u = 0; u < kU; u++) lv[u] = j0 + kT * u < end ? p[j0 + kT * u] : NAN;
+    for (int i = threadIdx.x; i < kBinWaves * tg.NB; i += kT) hist[i] = (T)0;
+    if (threadIdx.x < 64) {
+        const Stat s = wave_best(stats + ((uint64_t)b * g.R + row) * g.C, g.C);
+        const float sc = wave_bin_scale(reinterpret_cast<const Moments *>(ra), g.C, s.v, t, tg.NB);
+        if (threadIdx.x == 0) {
+            mx_s = s.v;
+            scale_s = sc;
+        }
+    }
+    __syncthreads();
+    const float mx = mx_s, scale = scale_s;
+    const int d = !COUNT && row < g.k ? drafts[(uint64_t)b * g.ds + row] : -1;
+    T *mine = hist + (threadIdx.x >> 6) * tg.NB;
+    while (j0 < end) {
+        float nx[kU];
+        const int jn = j0 + kU * kT;
+#pragma unroll
+        for (int u = 0; u < kU; u++) nx[u] = jn + kT * u < end ? p[jn + kT * u] : NAN;
+        if constexpr (COUNT) {
+#pragma unroll
+            for (int u = 0; u < kU; u++)
+                if (valid_logit(lv[u])) atomicAdd(&mine[bin_of(lv[u], mx, scale, tg.NB)], 1u);
+        } else {
+            // four weights at a time without branches: their chains of
+            // dependent float64 operations interleave
+            constexpr int kW = 4;
+#pragma unroll
+            for (int u0 = 0; u0 < kU; u0 += kW) {
+                double w[kW];
+#pragma unroll
+                for (int u = 0; u < kW; u++) w[u] = exp_nonpos_tab(exponent_of(lv[u0 + u], mx, t), tab);
+#pragma unroll
+                for (int u = 0; u < kW; u++) {
+                    const float l = lv[u0 + u];
+                    if (valid_logit(l) && j0 + kT * (u0 + u) != d)
+                        unsafeAtomicAdd(&mine[bin_of(l, mx, scale, tg.NB)], w[u]);
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kU; u++) lv[u] = nx[u];
+        j0 = jn;
+    }
+    __syncthreads();
+    T *out = reinterpret_cast<T *>(ra + tg.bins_off) + (uint64_t)c * tg.NB;
+    for (int i = threadIdx.x; i < tg.NB; i += kT) {
+        T v = hist[i];
+#pragma unroll
+        for (int w = 1; w < kBinWaves; w++) v += hist[w * tg.NB + i];
+        out[i] = v;
+    }
+}
+
+// The boundary bin of a row — the first where the members reach top_k
+// (COUNT) or the weight reaches the top_p share — and the chunk's members of
+// it (COUNT: of it and the bins above), each wave into its own segment in
+// (iteration, lane) order. Every workgroup of a row finds the boundary again
+// (a few KB from L2); the first one writes it down.
+template <bool COUNT>
+__global__ __launch_bounds__(256) void accept_collect_kernel(const float *__restrict__ logits, Geo g, TruncGeo tg,
+                                                             const int32_t *__restrict__ drafts,
+                                                             const Stat *__restrict__ stats, int top_k, float top_p,
+                                                             Temp t, uint8_t *__restrict__ area) {
+    using T = typename std::conditional<COUNT, uint32_t, double>::type;
+    __shared__ float mx_s, scale_s;
+    __shared__ int best_i_s, bnd_s;
+    __shared__ T wave_tot[4];
+    __shared__ T before_s;
+    const int c = blockIdx.x, row = blockIdx.y, b = blockIdx.z;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const float *p = row_ptr(logits, g, b, row);
+    uint8_t *ra = row_area(area, g, b, row);
+    // thread i owns bins [per i, per i + per): the chunks' sums in chunk order
+    constexpr int kPer = kBins / 256;
+    const int per = max(1, tg.NB / 256), lo = (int)threadIdx.x * per;
+    T h[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; i++) h[i] = (T)0;
+    const T *hist = reinterpret_cast<const T *>(ra + tg.bins_off);
+    for (int ch = 0; ch < tg.HC; ch++)
+#pragma unroll
+        for (int i = 0; i < kPer; i++)
+            if (i < per && lo + i < tg.NB) h[i] += hist[(uint64_t)ch * tg.NB + lo + i];
+    if (threadIdx.x < 64) {
+        const Stat s = wave_best(stats + ((uint64_t)b * g.R + row) * g.C, g.C);
+        const float sc = wave_bin_scale(reinterpret_cast<const Moments *>(ra), g.C, s.v, t, tg.NB);
+        if (threadIdx.x == 0) {
+            mx_s = s.v;
+            scale_s = sc;
+            best_i_s = s.i;
+            bnd_s = tg.NB;
+            before_s = (T)0;
+        }
+    }
+    T sum = (T)0;
+#pragma unroll
+    for (int i = 0; i < kPer; i++) sum += h[i];
+    T inc = sum;  // inclusive prefix over the wave
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const T v = __shfl_up(inc, off);
+        if (lane >= off) inc += v;
+    }
+    T exc = __shfl_up(inc, 1);
+    if (lane == 0) exc = (T)0;
+    if (lane == 63) wave_tot[wave] = inc;
+    __syncthreads();
+    const float mx = mx_s, scale = scale_s;
+    T tot = (T)0;
+    for (int w = 0; w < 4; w++) {
+        if (w == wave) exc += tot;
+        tot += wave_tot[w];
+    }
+    // the draft's own weight and bin
+    const int d = row < g.k ? drafts[(uint64_t)b * g.ds + row] : -1;
+    double wd = 0.0;
+    int dbin = tg.NB;
+    if (!COUNT && d >= 0 && d < g.V && valid_logit(p[d])) {
+        wd = soft_weight(p[d], mx, t);
+        dbin = bin_of(p[d], mx, scale, tg.NB);
+    }
+    const double total = (double)tot + wd;
+    {
+        T cum = exc;
+        int pick = -1;
+        T before = (T)0;
+#pragma unroll
+        for (int i = 0; i < kPer; i++) {
+            if (i >= per || lo + i >= tg.NB || pick >= 0) continue;
+            const T next = cum + h[i];
+            bool hit;
+            if constexpr (COUNT) hit = next >= (uint32_t)top_k;
+            else hit = next + (lo + i >= dbin ? wd : 0.0) >= (double)top_p * total && (h[i] > 0.0 || lo + i == dbin);
+            if (hit) {
+                pick = lo + i;
+                before = cum;
+            }
+            cum = next;
+        }
+        if (pick >= 0) atomicMin(&bnd_s, pick);
+        __syncthreads();
+        if (pick >= 0 && bnd_s == pick) before_s = before;
+    }
+    __syncthreads();
+    const int bnd = bnd_s;
+    int status = kCutFound;
+    if (COUNT) {
+        if (tot <= (T)top_k || bnd >= tg.NB - 1) status = kCutRow;
+    } else {
+        if (!(total > 0.0) || isinf(total) || bnd >= tg.NB) status = kCutAll;
+        else if (bnd == tg.NB - 1) status = kCutRow;
+    }
+    if (c == 0 && threadIdx.x == 0) {
+        RowCut &o = row_cut(area, g, b, row);
+        o.cut = Cut{0u, INT_MAX};
+        o.rest = (double)tot;  // (kCutAll)
+        o.wd = wd;
+        o.total = total;
+        o.before = (double)before_s + (dbin < bnd ? wd : 0.0);
+        o.before_rest = (double)before_s;
+        o.best_v = mx;
+        o.best_i = best_i_s;
+        o.status = status;
+    }
+    const int w = c * 4 + wave;
+    uint32_t found = 0u;
+    if (status == kCutFound) {
+        Member *out = reinterpret_cast<Member *>(ra + tg.cand_off) + (uint64_t)w * tg.seg;
+        const int begin = (int)((int64_t)g.V * c / tg.KC), end = (int)((int64_t)g.V * (c + 1) / tg.KC);
+        constexpr int kU = 8;
+        for (int j0 = begin + threadIdx.x; j0 - (int)threadIdx.x < end; j0 += kU * 256) {
+            float l[kU];
+#pragma unroll
+            for (int u = 0; u < kU; u++) l[u] = j0 + 256 * u < end ? p[j0 + 256 * u] : NAN;
+#pragma unroll
+            for (int u = 0; u < kU; u++) {
+                const int bin = bin_of(l[u], mx, scale, tg.NB);
+                const bool take = valid_logit(l[u]) && (COUNT ? bin <= bnd : bin == bnd);
+                const uint64_t m = __ballot(take);
+                if (!m) continue;
+                const uint32_t at = found + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+                if (take && at < (uint32_t)tg.seg) out[at] = Member{l[u], j0 + 256 * u};
+                found += (uint32_t)__popcll(m);
+            }
+        }
+    }
+    if (lane == 0) reinterpret_cast<uint32_t *>(ra + tg.cnt_off)[w] = found;
+}
+
+// ---- exact cut among a row's elements or its candidates: radix selection
+// over the 32-bit order key, histograms in LDS. Each wave fills its own
+// histogram and the waves are combined in wave order, so weight sums do not
+// depend on wave scheduling.
 constexpr int kSelWaves = 16;
 
 struct SelShared {
@@ -236,94 +665,56 @@ struct SelShared {
     double total_w;     // all weight of the first pass
     uint32_t total_c;
     int id;             // result of an id selection
-    float mx;
 };
 
-// Top-p candidates held in LDS (dynamic shared memory of the select kernel):
-// the ids of the first digit's boundary bucket, collected by the second pass
-// when they fit, so that the third and fourth digits read those logits
-// (from L2: the second pass has just read the row) instead of the row. Each
-// wave fills its own segment in a fixed order, so the later passes add the
-// same values in the same order on every run.
-constexpr int kCandCap = 24576;
-constexpr int kCandWave = kCandCap / kSelWaves;  // per-wave segment
-struct Cands {
-    int *j;       // [wave][kCandWave]
-    uint32_t *n;  // [wave] candidates found (more than kCandWave: not all stored)
+// The elements a selection runs over: a candidate list in LDS, or (list
+// null) the whole row.
+struct SelSrc {
+    const float *p;
+    int V;
+    const Member *list;
+    int n;
+    bool top;  // the list is the row's top, top_k members or more
 };
 
-// Histogram of the next digit over the row's elements that `sel` admits;
-// with C, the admitted elements are also appended to the candidate list.
-template <bool W, bool C = false, class Sel, class Dig>
-__device__ __forceinline__ void hist_pass(const float *__restrict__ p, int V, float mx, double t, SelShared &s,
-                                          Sel sel, Dig dig, Cands cand = Cands{nullptr, nullptr}) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    for (int b = lane; b < 256; b += 64) {
-        s.cnt[wave][b] = 0u;
-        if (W) s.wsum[wave][b] = 0.0;
-    }
-    __syncthreads();
+// f(logit, id) for every valid element, in a fixed order per thread.
+template <class F>
+__device__ __forceinline__ void for_each(const SelSrc &src, F f) {
     constexpr int kStride = kSelWaves * 64;
+    if (src.list) {
+        for (int i = threadIdx.x; i < src.n; i += kStride)
+            if (valid_logit(src.list[i].l)) f(src.list[i].l, src.list[i].j);
+        return;
+    }
     // eight loads in flight per thread (the row is read from L2 / the
     // Infinity Cache once per pass: latency, not bandwidth, bounds the pass)
     constexpr int kU = 8;
-    uint32_t wn = 0u;  // candidates of this wave so far
-    for (int j0 = threadIdx.x; j0 < V; j0 += kU * kStride) {
+    for (int j0 = threadIdx.x; j0 < src.V; j0 += kU * kStride) {
         float l[kU];
 #pragma unroll
-        for (int u = 0; u < kU; u++) l[u] = j0 + u * kStride < V ? p[j0 + u * kStride] : NAN;
+        for (int u = 0; u < kU; u++) l[u] = j0 + u * kStride < src.V ? src.p[j0 + u * kStride] : NAN;
 #pragma unroll
-        for (int u = 0; u < kU; u++) {
-            const int j = j0 + u * kStride;
-            const bool take = valid_logit(l[u]) && sel(l[u], j);
-            if (C) {
-                // this wave's segment, in (iteration, lane) order: the list is
-                // the same on every run, whatever the waves' timing
-                const uint64_t m = __ballot(take);
-                const uint32_t at = wn + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-                if (take && at < (uint32_t)kCandWave) cand.j[wave * kCandWave + at] = j;
-                wn += (uint32_t)__popcll(m);
-            }
-            if (!take) continue;
-            const int b = dig(l[u], j);
-            atomicAdd(&s.cnt[wave][b], 1u);
-            if (W) unsafeAtomicAdd(&s.wsum[wave][b], exp((double)(l[u] - mx) / t));
-        }
+        for (int u = 0; u < kU; u++)
+            if (valid_logit(l[u])) f(l[u], j0 + u * kStride);
     }
-    if (C && lane == 0) cand.n[wave] = wn;
-    __syncthreads();
-    if (threadIdx.x < 256) {
-        uint32_t c = 0u;
-        double w = 0.0;
-        for (int q = 0; q < kSelWaves; q++) {
-            c += s.cnt[q][threadIdx.x];
-            if (W) w += s.wsum[q][threadIdx.x];
-        }
-        s.tc[threadIdx.x] = c;
-        s.tw[threadIdx.x] = w;
-    }
-    __syncthreads();
 }
 
-// hist_pass over the candidate list instead of the row.
-template <bool W, class Sel, class Dig>
-__device__ __forceinline__ void hist_cands(const float *__restrict__ p, const Cands cand, float mx, double t,
-                                           SelShared &s, Sel sel, Dig dig) {
+// Histogram of the next digit over the elements that `sel` admits.
+template <bool W, class Sel>
+__device__ __forceinline__ void hist_pass(const SelSrc &src, float mx, const Temp &t, SelShared &s, int shift, Sel sel) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for (int b = lane; b < 256; b += 64) {
         s.cnt[wave][b] = 0u;
         if (W) s.wsum[wave][b] = 0.0;
     }
     __syncthreads();
-    const uint32_t n = min(cand.n[wave], (uint32_t)kCandWave);  // (the caller checked every segment fits)
-    for (uint32_t i = lane; i < n; i += 64) {  // wave w walks segment w
-        const int j = cand.j[wave * kCandWave + i];
-        const float l = p[j];
-        if (!sel(l, j)) continue;
-        const int b = dig(l, j);
+    for_each(src, [&](float l, int j) __attribute__((always_inline)) {
+        const uint32_t k = order_key(l);
+        if (!sel(k, j)) return;
+        const int b = (k >> shift) & 255u;
         atomicAdd(&s.cnt[wave][b], 1u);
-        if (W) unsafeAtomicAdd(&s.wsum[wave][b], exp((double)(l - mx) / t));
-    }
+        if (W) unsafeAtomicAdd(&s.wsum[wave][b], soft_weight(l, mx, t));
+    });
     __syncthreads();
     if (threadIdx.x < 256) {
         uint32_t c = 0u;
@@ -468,100 +859,13 @@ __device__ int select_id(const float *p, int V, SelShared &s, uint32_t key, Cut 
     return id;
 }
 
-// First top-p digit of one chunk of a row: counts and weights of the
-// elements inside the top-k cut by the top byte of their order key. One
-// workgroup per (chunk, row, request), so the float64 exponentials of the
-// whole vocabulary spread over the GPU; the select kernel adds the chunks in
-// chunk order (deterministic).
-struct Hist0 {
-    uint32_t c[256];
-    double w[256];
-};
-
-__global__ __launch_bounds__(256) void accept_hist_kernel(const float *__restrict__ logits, Geo g,
-                                                          const Stat *__restrict__ stats,
-                                                          const Cut *__restrict__ cuts, double t,
-                                                          Hist0 *__restrict__ out) {
-    const int c = blockIdx.x, row = blockIdx.y, b = blockIdx.z;
-    const int wave = threadIdx.x >> 6;
-    const float *p = row_ptr(logits, g, b, row);
-    __shared__ float mx_s;
-    __shared__ uint32_t cnt[4][256];
-    __shared__ double ws[4][256];
-    for (int i = threadIdx.x; i < 4 * 256; i += 256) {
-        (&cnt[0][0])[i] = 0u;
-        (&ws[0][0])[i] = 0.0;
-    }
-    if (threadIdx.x < 64) {  // wave 0 reduces the row's chunk maxima
-        const Stat *st = stats + ((uint64_t)b * g.R + row) * g.C;
-        float bv = -INFINITY;
-        int bi = INT_MAX;
-        for (int cc = threadIdx.x; cc < g.C; cc += 64)
-            if (beats(st[cc].v, st[cc].i, bv, bi)) { bv = st[cc].v; bi = st[cc].i; }
-        for (int off = 32; off > 0; off >>= 1) {
-            const float ov = __shfl_xor(bv, off);
-            const int oi = __shfl_xor(bi, off);
-            if (beats(ov, oi, bv, bi)) { bv = ov; bi = oi; }
-        }
-        if (threadIdx.x == 0) mx_s = bv;
-    }
-    __syncthreads();
-    const float mx = mx_s;
-    const Cut cut = row_cut(cuts, g, b, row);
-    const int begin = c * g.L, end = min(begin + g.L, g.V);
-    constexpr int kU = 8;  // loads in flight per thread
-    for (int j0 = begin + threadIdx.x; j0 < end; j0 += kU * 256) {
-        float lv[kU];
-#pragma unroll
-        for (int u = 0; u < kU; u++) lv[u] = j0 + 256 * u < end ? p[j0 + 256 * u] : NAN;
-#pragma unroll
-        for (int u = 0; u < kU; u++) {
-            const int j = j0 + 256 * u;
-            const float l = lv[u];
-            if (!valid_logit(l)) continue;
-            const uint32_t k = order_key(l);
-            if (!in_cut(k, j, cut)) continue;
-            atomicAdd(&cnt[wave][k >> 24], 1u);
-            unsafeAtomicAdd(&ws[wave][k >> 24], exp((double)(l - mx) / t));
-        }
-    }
-    __syncthreads();
-    Hist0 &o = out[((uint64_t)b * g.R + row) * g.C + c];
-    const int q = threadIdx.x;
-    o.c[q] = cnt[0][q] + cnt[1][q] + cnt[2][q] + cnt[3][q];
-    o.w[q] = ((ws[0][q] + ws[1][q]) + ws[2][q]) + ws[3][q];
-}
-
-// mode 0: top-k then top-p in one launch; 1: top-k only; 2: top-p only, the
-// top-k cut (top_k > 0) read from `cuts` and the first digit's histogram
-// summed from accept_hist_kernel's chunks.
-__global__ __launch_bounds__(1024) void accept_select_kernel(const float *__restrict__ logits, Geo g,
-                                                             const Stat *__restrict__ stats, int top_k,
-                                                             float top_p, double t, Cut *__restrict__ cuts,
-                                                             int mode, const Hist0 *__restrict__ h0) {
-    const int row = blockIdx.x, b = blockIdx.y;
-    const float *p = row_ptr(logits, g, b, row);
-    __shared__ SelShared s;
-    if (threadIdx.x < 64) {  // the row maximum from the per-chunk statistics
-        const Stat *st = stats + ((uint64_t)b * g.R + row) * g.C;
-        float bv = -INFINITY;
-        int bi = INT_MAX;
-        for (int cc = threadIdx.x; cc < g.C; cc += 64)
-            if (beats(st[cc].v, st[cc].i, bv, bi)) { bv = st[cc].v; bi = st[cc].i; }
-        for (int off = 32; off > 0; off >>= 1) {
-            const float ov = __shfl_xor(bv, off);
-            const int oi = __shfl_xor(bi, off);
-            if (beats(ov, oi, bv, bi)) { bv = ov; bi = oi; }
-        }
-        if (threadIdx.x == 0) s.mx = bv;
-    }
-    __syncthreads();
-    const float mx = s.mx;
+// The cut of one row by radix selection over src. With `tail` (candidates of
+// one bin): the weight `before` lies ahead of src's elements, of `total`.
+__device__ __forceinline__ Cut radix_cut(const SelSrc src, SelShared &s, float mx, const Temp t, int top_k, float top_p,
+                                         bool tail, double before, double total) {
     Cut cut{0u, INT_MAX};
-    if (mode == 2 && top_k > 0) cut = cuts[(uint64_t)b * g.R + row];
-
     // top-k: the top_k-th element in (logit desc, id asc) order (sampling.go:90-92).
-    if (top_k > 0 && mode != 2) {
+    if (top_k > 0) {
         if (threadIdx.x == 0) {
             s.prefix = 0u;
             s.before_c = 0u;
@@ -573,9 +877,7 @@ __global__ __launch_bounds__(1024) void accept_select_kernel(const float *__rest
             const int shift = 24 - 8 * pass;
             const uint32_t mask = pass ? ~0u << (shift + 8) : 0u;
             const uint32_t pre = s.prefix;
-            hist_pass<false>(
-                p, g.V, mx, t, s, [=](float l, int) { return (order_key(l) & mask) == pre; },
-                [=](float l, int) { return (order_key(l) >> shift) & 255u; });
+            hist_pass<false>(src, mx, t, s, shift, [=](uint32_t k, int) { return (k & mask) == pre; });
             if (threadIdx.x < 64) {
                 uint32_t tot_c = s.total_c;
                 if (pass == 0) {
@@ -583,10 +885,10 @@ __global__ __launch_bounds__(1024) void accept_select_kernel(const float *__rest
                     bucket_totals(s, &tot_c, &unused);
                     if (threadIdx.x == 0) s.total_c = tot_c;
                 }
-                if (tot_c > (uint32_t)top_k) scan_buckets(s, true, false, (uint32_t)top_k, 0.0, shift);
+                if (src.top || tot_c > (uint32_t)top_k) scan_buckets(s, true, false, (uint32_t)top_k, 0.0, shift);
             }
             __syncthreads();
-            if (s.total_c <= (uint32_t)top_k) {
+            if (!src.top && s.total_c <= (uint32_t)top_k) {
                 all = true;
                 break;
             }
@@ -597,65 +899,34 @@ __global__ __launch_bounds__(1024) void accept_select_kernel(const float *__rest
             const uint32_t ties = s.tc[s.bucket];
             __syncthreads();
             cut.key = key;
-            cut.id = need < ties ? select_id(p, g.V, s, key, Cut{0u, INT_MAX}, need) : INT_MAX;
+            cut.id = need < ties ? select_id(src.p, src.V, s, key, Cut{0u, INT_MAX}, need) : INT_MAX;
         }
     }
 
     // top-p: the smallest prefix whose cumulative share reaches top_p
     // (sampling.go:104-113), within the top-k set.
-    if (top_p > 0.0f && top_p < 1.0f && mode != 1) {
+    if (top_p > 0.0f && top_p < 1.0f) {
         __syncthreads();
         if (threadIdx.x == 0) {
             s.prefix = 0u;
             s.before_c = 0u;
-            s.before_w = 0.0;
+            s.before_w = tail ? before : 0.0;
         }
         __syncthreads();
         bool found = true;
-        // mode 2: the second pass keeps the first digit's bucket in LDS when
-        // it fits; the later passes then scan only those elements
-        extern __shared__ uint8_t sel_dyn[];
-        const Cands cand{reinterpret_cast<int *>(sel_dyn), reinterpret_cast<uint32_t *>(sel_dyn + kCandCap * 4)};
-        bool compact = false;
         for (int pass = 0; pass < 4 && found; pass++) {
             const int shift = 24 - 8 * pass;
             const uint32_t mask = pass ? ~0u << (shift + 8) : 0u;
             const uint32_t pre = s.prefix;
             const Cut ck = cut;
-            const auto sel_fn = [=](float l, int j) {
-                const uint32_t k = order_key(l);
-                return in_cut(k, j, ck) && (k & mask) == pre;
-            };
-            const auto dig_fn = [=](float l, int) { return (order_key(l) >> shift) & 255u; };
-            const bool collect = mode == 2 && pass == 1 && s.tc[s.bucket] <= (uint32_t)kCandCap;
-            if (pass == 0 && h0) {  // chunk histograms, added in chunk order
-                if (threadIdx.x < 256) {
-                    const Hist0 *hr = h0 + ((uint64_t)b * g.R + row) * g.C;
-                    uint32_t cc = 0u;
-                    double w = 0.0;
-                    for (int ch = 0; ch < g.C; ch++) {
-                        cc += hr[ch].c[threadIdx.x];
-                        w += hr[ch].w[threadIdx.x];
-                    }
-                    s.tc[threadIdx.x] = cc;
-                    s.tw[threadIdx.x] = w;
-                }
-                __syncthreads();
-            } else if (compact) {
-                hist_cands<true>(p, cand, mx, t, s, sel_fn, dig_fn);
-            } else if (collect) {
-                hist_pass<true, true>(p, g.V, mx, t, s, sel_fn, dig_fn, cand);
-                bool fits = true;
-                for (int w = 0; w < kSelWaves; w++) fits = fits && cand.n[w] <= (uint32_t)kCandWave;
-                compact = fits;  // else the later digits read the row
-            } else {
-                hist_pass<true>(p, g.V, mx, t, s, sel_fn, dig_fn);
-            }
+            hist_pass<true>(src, mx, t, s, shift,
+                            [=](uint32_t k, int j) { return in_cut(k, j, ck) && (k & mask) == pre; });
             if (threadIdx.x < 64) {
                 double tot = s.total_w;
                 if (pass == 0) {
                     uint32_t unused;
                     bucket_totals(s, &unused, &tot);
+                    if (tail) tot = total;
                     if (threadIdx.x == 0) s.total_w = tot;
                 }
                 if (tot > 0.0 && !isinf(tot))
@@ -673,7 +944,7 @@ __global__ __launch_bounds__(1024) void accept_select_kernel(const float *__rest
                 const uint32_t key = s.prefix;
                 const uint32_t ties = s.tc[s.bucket];
                 const double tot = s.total_w;
-                const double wt = exp((double)(key_value(key) - mx) / t);
+                const double wt = soft_weight(key_value(key), mx, t);
                 double cum = s.before_w / tot;
                 uint32_t m = ties;
                 for (uint32_t i = 1; i <= ties; i++) {
@@ -690,11 +961,166 @@ __global__ __launch_bounds__(1024) void accept_select_kernel(const float *__rest
             const uint32_t key = s.prefix, m = s.before_c, ties = s.total_c;
             __syncthreads();
             Cut nc{key, key == cut.key ? cut.id : INT_MAX};
-            if (m < ties) nc.id = select_id(p, g.V, s, key, cut, m);
+            if (m < ties) nc.id = select_id(src.p, src.V, s, key, cut, m);
             cut = nc;
         }
     }
-    if (threadIdx.x == 0) cuts[(uint64_t)b * g.R + row] = cut;
+    return cut;
+}
+
+// Sum over the workgroup in wave order, in every thread.
+__device__ __forceinline__ double block_sum(double v, double *waves) {
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) waves[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double t = 0.0;
+    for (int w = 0; w < kSelWaves; w++) t += waves[w];
+    return t;
+}
+
+// One workgroup per row: the exact cut, and the kept weight without the
+// draft and of the draft. Up to kRankMost candidates are put in order by
+// counting (thread i adds up what lies ahead of candidate i); more take the
+// radix selection. `direct`: no candidates were collected, the row itself is
+// taken (into LDS).
+__global__ __launch_bounds__(64 * kSelWaves) void accept_cut_kernel(const float *__restrict__ logits, Geo g, TruncGeo tg,
+                                                                    const int32_t *__restrict__ drafts,
+                                                                    const Stat *__restrict__ stats, int top_k, float top_p,
+                                                                    Temp t, uint8_t *__restrict__ area, int direct) {
+    const int row = blockIdx.x, b = blockIdx.y;
+    const float *p = row_ptr(logits, g, b, row);
+    uint8_t *ra = row_area(area, g, b, row);
+    RowCut &rc = row_cut(area, g, b, row);
+    __shared__ SelShared s;
+    __shared__ double waves[kSelWaves];
+    __shared__ uint32_t seg_at[260];
+    __shared__ unsigned long long cut_s;
+    __shared__ int n_s;
+    extern __shared__ __attribute__((aligned(16))) uint8_t cut_dyn[];
+    Member *list = reinterpret_cast<Member *>(cut_dyn);
+    RowCut in = rc;
+    if (direct) {
+        __shared__ Stat best_s;
+        for (int j = threadIdx.x; j < g.V; j += 64 * kSelWaves) list[j] = Member{p[j], j};
+        if (threadIdx.x < 64) {
+            const Stat best = wave_best(stats + ((uint64_t)b * g.R + row) * g.C, g.C);
+            if (threadIdx.x == 0) best_s = best;
+        }
+        __syncthreads();
+        in.status = kCutRow;
+        in.best_v = best_s.v;
+        in.best_i = best_s.i;
+    }
+    const float mx = in.best_v;
+    if (in.status == kCutAll) return;  // the defaults of collect hold
+    const int d = row < g.k ? drafts[(uint64_t)b * g.ds + row] : -1;
+    bool fits = in.status == kCutFound;
+    const int segs = tg.KC * 4;
+    if (fits) {  // segment starts (wave 0: up to 256 segments, 4 a lane), then the members side by side
+        if (threadIdx.x < 64) {
+            const uint32_t *cnt = reinterpret_cast<const uint32_t *>(ra + tg.cnt_off);
+            uint32_t c[4], sum = 0u;
+            bool ok = true;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int q = 4 * (int)threadIdx.x + i;
+                c[i] = q < segs ? cnt[q] : 0u;
+                ok = ok && c[i] <= (uint32_t)tg.seg;
+                sum += c[i];
+            }
+            uint32_t inc = sum;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const uint32_t v = __shfl_up(inc, off);
+                if ((int)threadIdx.x >= off) inc += v;
+            }
+            uint32_t at = inc - sum;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                seg_at[4 * threadIdx.x + i] = at;
+                at += c[i];
+            }
+            if (threadIdx.x == 63) seg_at[256] = at;
+            const uint64_t good = __ballot(ok);
+            if (threadIdx.x == 63) n_s = good == ~0ull && at <= (uint32_t)kCandMost ? (int)at : -1;
+        }
+        __syncthreads();
+        fits = n_s >= 0;
+    }
+    if (fits) {
+        const Member *src = reinterpret_cast<const Member *>(ra + tg.cand_off);
+        for (int q = threadIdx.x >> 6; q < segs; q += kSelWaves) {
+            const uint32_t a = seg_at[q], n = seg_at[q + 1] - a;
+            for (uint32_t i = threadIdx.x & 63; i < n; i += 64) list[a + i] = src[(uint64_t)q * tg.seg + i];
+        }
+        __syncthreads();
+    }
+    const int n = fits ? n_s : 0;
+    Cut cut{0u, INT_MAX};
+    if (fits && n <= kRankMost) {
+        // composite order: a larger (key, ~id) is ahead
+        unsigned long long *ord = reinterpret_cast<unsigned long long *>(&s.wsum[0][0]);
+        double *wt = reinterpret_cast<double *>(&s.wsum[0][0]) + kRankMost;
+        const int i = threadIdx.x;
+        const bool have = i < n;
+        const unsigned long long me =
+            have ? ((unsigned long long)order_key(list[i].l) << 32) | (uint32_t)~(uint32_t)list[i].j : 0ull;
+        double w = 0.0;
+        if (have) ord[i] = me;
+        if (threadIdx.x == 0) cut_s = ~0ull;
+        __syncthreads();
+        bool keep = have;
+        if (top_k > 0) {  // the candidates are everything down to the boundary bin
+            uint32_t ahead = 0u;
+            for (int q = 0; q < n; q++) ahead += ord[q] > me;
+            keep = have && ahead < (uint32_t)top_k;
+        }
+        if (keep) w = soft_weight(list[i].l, mx, t);
+        if (have) wt[i] = keep ? w : 0.0;
+        double total = in.total, before = in.before;
+        if (top_k > 0) {
+            total = block_sum(w, waves);
+            before = 0.0;
+        }
+        __syncthreads();
+        // the last kept member: the first one whose running share reaches
+        // top_p, else the lowest kept one
+        const bool nucleus = top_p > 0.0f && top_p < 1.0f && total > 0.0 && !isinf(total);
+        bool reach = false;
+        if (nucleus) {
+            double ahead = 0.0;
+            for (int q = 0; q < n; q++) ahead += ord[q] > me ? wt[q] : 0.0;
+            reach = keep && before + ahead + w >= (double)top_p * total;
+        }
+        // (a first reach is the largest composite among those that reach)
+        __shared__ unsigned long long first_s;
+        if (threadIdx.x == 0) first_s = 0ull;
+        __syncthreads();
+        if (reach) atomicMax(&first_s, me);
+        if (keep) atomicMin(&cut_s, me);
+        __syncthreads();
+        const unsigned long long last = first_s ? first_s : cut_s;
+        cut = Cut{(uint32_t)(last >> 32), (int32_t)~(uint32_t)last};
+    } else {
+        const SelSrc src{p, g.V, fits || direct ? list : nullptr, fits ? n : g.V, fits && top_k > 0};
+        cut = radix_cut(src, s, mx, t, top_k, top_p, fits && top_k <= 0, in.before, in.total);
+        __syncthreads();
+    }
+    // the kept weight: candidates (after the bins above them), or the row
+    const SelSrc src{p, g.V, fits || direct ? list : nullptr, fits ? n : g.V, false};
+    double sum = 0.0;
+    for_each(src, [&](float l, int j) __attribute__((always_inline)) {
+        if (j != d && in_cut(order_key(l), j, cut)) sum += soft_weight(l, mx, t);
+    });
+    sum = block_sum(sum, waves);
+    if (threadIdx.x == 0) {
+        rc.best_v = in.best_v;
+        rc.best_i = in.best_i;
+        rc.cut = cut;
+        rc.rest = sum + (fits && top_k <= 0 ? in.before_rest : 0.0);
+        rc.wd = d >= 0 && d < g.V ? weight_of(p[d], d, mx, t, cut) : 0.0;
+    }
 }
 
 // Philox4x32-10 (Salmon et al., SC'11).
@@ -741,14 +1167,12 @@ __global__ __launch_bounds__(256) void router_normal_kernel(float *__restrict__ 
     if (2 * p + 1 < E) row[2 * p + 1] = (float)(rad * sin(ang));
 }
 
-// Block-wide inverse CDF inside chunk `c` of a row: the first index j (j != d,
+// Block-wide inverse CDF inside the chunk [begin, end) of a row: the first index j (j != d,
 // weight > 0) whose running weight sum exceeds `target`. Returns -1 when the
 // target lies beyond the chunk's own sum (rounding), with *last the last
 // positive-weight index of the chunk.
-__device__ int scan_chunk(const float *p, const Geo &g, int c, int d, float mx, double t, const Cut &cut,
+__device__ int scan_chunk(const float *p, int begin, int end, int d, float mx, const Temp &t, const Cut &cut,
                           double target, double *shared_prefix, int *shared_pick) {
-    const int begin = c * g.L;
-    const int end = min(begin + g.L, g.V);
     const int len = end - begin;
     const int per = (len + 255) / 256;
     const int lo = begin + threadIdx.x * per;
@@ -809,8 +1233,7 @@ __device__ int scan_chunk(const float *p, const Geo &g, int c, int d, float mx, 
 __global__ __launch_bounds__(256) void accept_finalize_kernel(
     const float *__restrict__ logits, Geo g, const int32_t *__restrict__ drafts,
     const Stat *__restrict__ stats, const double *__restrict__ sums,
-    const double *__restrict__ wdraft, const Cut *__restrict__ cuts, int stochastic, double t, uint64_t seed,
-    uint64_t step,
+    const double *__restrict__ wdraft, int stochastic, Temp t, uint64_t seed, uint64_t step,
     uint32_t request_base, int32_t *__restrict__ result, double *__restrict__ debug,
     const uint64_t *__restrict__ step_dev, const int32_t *__restrict__ forced) {
     const int b = blockIdx.x;
@@ -951,7 +1374,8 @@ __global__ __launch_bounds__(256) void accept_finalize_kernel(
         }
         if (action == 2) {
             const int d = row < g.k ? drafts[(uint64_t)b * g.ds + row] : -1;
-            const int j = scan_chunk(p, g, cstar, d, mx_s, t, row_cut(cuts, g, b, row), target_s, prefix, &pick);
+            const int begin = cstar * g.L;
+            const int j = scan_chunk(p, begin, min(begin + g.L, g.V), d, mx_s, t, Cut{0u, INT_MAX}, target_s, prefix, &pick);
             if (threadIdx.x == 0) decided_next = j >= 0 ? j : best_s.i;
         }
         break;
@@ -962,6 +1386,173 @@ __global__ __launch_bounds__(256) void accept_finalize_kernel(
         o[0] = accepted_s;
         o[1] = decided_next;
         o[2] = argmax0;
+        o[3] = 0;
+    }
+}
+
+// What the rows of a request decide (truncated stochastic acceptance):
+// the first row that does not accept its draft, and what follows there.
+struct Decision {
+    int row;       // rows accepted
+    int next;      // the next token, or -1: drawn from `row`
+    double target; // of the draw: a share of the row's kept weight in index order
+    int d;         // draft left out of the draw (-1: none)
+};
+
+// Wave 0 of a workgroup: lane l takes rows l, l + 64, ...; every lane
+// returns the decision.
+__device__ Decision decide(const float *logits, const Geo &g, int b, const int32_t *drafts, uint8_t *area,
+                           uint64_t seed, uint64_t step, uint32_t request, const int32_t *forced, double *debug) {
+    const int lane = threadIdx.x & 63;
+    const int flen = forced ? forced[b] : -1;
+    for (int r0 = 0;; r0 += 64) {
+        const int row = r0 + lane;
+        bool stop = false, onehot = false;
+        double rest = 0.0, total = 0.0, pd = 0.0, u = 0.0;
+        Stat sb{-INFINITY, INT_MAX};
+        float shown = 0.f;
+        int d = -1;
+        if (row <= g.k) {
+            const RowCut &rc = row_cut(area, g, b, row);
+            sb = Stat{rc.best_v, rc.best_i};
+            rest = rc.rest;
+            total = rest + rc.wd;
+            onehot = !(total > 0.0) || isinf(total);
+            // argmaxLogit keeps a NaN at index 0; the sampler falls back to
+            // its answer when no logit is valid (sampling.go:83-89)
+            const float p0 = row_ptr(logits, g, b, row)[0];
+            shown = p0 != p0 ? p0 : sb.v;
+            if (sb.v == -INFINITY && p0 != p0) sb = Stat{p0, 0};
+            if (row < g.k) {
+                d = drafts[(uint64_t)b * g.ds + row];
+                pd = onehot ? (d == sb.i ? 1.0 : 0.0) : rc.wd / total;
+                u = draw(seed, step, (uint32_t)row, request, 0);
+                stop = !(forced ? row < flen : u < pd);
+            } else {
+                stop = true;
+            }
+        }
+        const uint64_t m = __ballot(stop);
+        const int first = m ? __ffsll((unsigned long long)m) - 1 : 64;
+        if (debug && row <= g.k && lane <= first) {
+            double *o = debug + ((uint64_t)b * g.R + row) * 4;
+            o[0] = pd;
+            o[1] = u;
+            o[2] = total;
+            o[3] = (double)shown;
+        }
+        if (!m) continue;
+        Decision dec{r0 + first, -1, 0.0, -1};
+        int next = -1;
+        double target = 0.0;
+        if (lane == first) {
+            if (onehot || (row < g.k && !(rest > 0.0)))
+                next = sb.i;
+            else
+                target = draw(seed, step, (uint32_t)row, request, 1) * (row < g.k ? rest : total);
+        }
+        dec.next = __shfl(next, first);
+        dec.target = __shfl(target, first);
+        dec.d = __shfl(d, first);
+        return dec;
+    }
+}
+
+// Kept weight per chunk of the row that a request draws from (RC chunks).
+__global__ __launch_bounds__(256) void accept_resample_kernel(const float *__restrict__ logits, Geo g, int RC,
+                                                              const int32_t *__restrict__ drafts,
+                                                              uint8_t *__restrict__ area, Temp t, uint64_t seed,
+                                                              uint64_t step, uint32_t request_base,
+                                                              const uint64_t *__restrict__ step_dev,
+                                                              const int32_t *__restrict__ forced,
+                                                              double *__restrict__ sums) {
+    const int c = blockIdx.x, b = blockIdx.y;
+    __shared__ int row_s, d_s;
+    __shared__ double ws[4];
+    if (step_dev) step = *step_dev;
+    if (threadIdx.x < 64) {
+        const Decision dec = decide(logits, g, b, drafts, area, seed, step, request_base + (uint32_t)b, forced, nullptr);
+        if (threadIdx.x == 0) {
+            row_s = dec.next < 0 ? dec.row : -1;
+            d_s = dec.d;
+        }
+    }
+    __syncthreads();
+    const int row = row_s, d = d_s;
+    if (row < 0) return;
+    const RowCut &rc = row_cut(area, g, b, row);
+    const Cut cut = rc.cut;
+    const float mx = rc.best_v;
+    const float *p = row_ptr(logits, g, b, row);
+    const int begin = (int)((int64_t)g.V * c / RC), end = (int)((int64_t)g.V * (c + 1) / RC);
+    double acc = 0.0;
+    constexpr int kU = 8;
+    for (int j0 = begin + threadIdx.x; j0 < end; j0 += kU * 256) {
+        float l[kU];
+#pragma unroll
+        for (int u = 0; u < kU; u++) l[u] = j0 + u * 256 < end ? p[j0 + u * 256] : NAN;
+#pragma unroll
+        for (int u = 0; u < kU; u++)
+            if (j0 + u * 256 != d) acc += weight_of(l[u], j0 + u * 256, mx, t, cut);
+    }
+    for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
+    if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) sums[(uint64_t)b * RC + c] = ws[0] + ws[1] + ws[2] + ws[3];
+}
+
+// The draw: the chunk that the target falls into, then the index inside it.
+__global__ __launch_bounds__(256) void accept_pick_kernel(const float *__restrict__ logits, Geo g, int RC,
+                                                          const int32_t *__restrict__ drafts,
+                                                          uint8_t *__restrict__ area,
+                                                          const double *__restrict__ sums, Temp t, uint64_t seed,
+                                                          uint64_t step, uint32_t request_base,
+                                                          const uint64_t *__restrict__ step_dev,
+                                                          const int32_t *__restrict__ forced,
+                                                          int32_t *__restrict__ result, double *__restrict__ debug) {
+    const int b = blockIdx.x, lane = threadIdx.x & 63;
+    __shared__ double prefix[256];
+    __shared__ int pick, cstar_s;
+    __shared__ double target_s;
+    __shared__ Decision dec_s;
+    if (step_dev) step = *step_dev;
+    if (threadIdx.x < 64) {
+        // RC <= 64: lane c's chunk; the target's chunk is the last one whose
+        // running start it reaches
+        const double cs = lane < RC ? sums[(uint64_t)b * RC + lane] : 0.0;
+        const Decision dec = decide(logits, g, b, drafts, area, seed, step, request_base + (uint32_t)b, forced, debug);
+        double inc = cs;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const double v = __shfl_up(inc, off);
+            if (lane >= off) inc += v;
+        }
+        const uint64_t m = __ballot(lane < RC - 1 && !(dec.target < inc));
+        const int c = m == ~0ull ? 63 : __ffsll((unsigned long long)~m) - 1;  // leading chunks that end at or before it
+        const double run = __shfl(inc, c ? c - 1 : 0);
+        if (lane == 0) {
+            dec_s = dec;
+            cstar_s = c;
+            target_s = dec.target - (c ? run : 0.0);
+        }
+    }
+    __syncthreads();
+    const Decision dec = dec_s;
+    int next = dec.next;
+    if (next < 0) {
+        const RowCut &rc = row_cut(area, g, b, dec.row);
+        const int c = cstar_s;
+        const int j = scan_chunk(row_ptr(logits, g, b, dec.row), (int)((int64_t)g.V * c / RC),
+                                 (int)((int64_t)g.V * (c + 1) / RC), dec.d, rc.best_v, t, rc.cut, target_s, prefix, &pick);
+        next = j >= 0 ? j : rc.best_i;
+    }
+    if (threadIdx.x == 0) {
+        // argmaxLogit of row 0 keeps a NaN at index 0
+        const float p0 = row_ptr(logits, g, b, 0)[0];
+        int32_t *o = result + (uint64_t)b * 4;
+        o[0] = dec.row;
+        o[1] = next;
+        o[2] = p0 != p0 ? 0 : row_cut(area, g, b, 0).best_i;
         o[3] = 0;
     }
 }
@@ -983,13 +1574,31 @@ Geo make_geo(const yuuka_accept_params &p) {
     return g;
 }
 
+// The layout of a row's area. The bins take at most about half of it, the
+// candidates the rest; few rows have many chunks and much room, thousands of
+// rows little (fewer bins, and more of their rows scan the row).
+TruncGeo trunc_geo(const Geo &g) {
+    TruncGeo t;
+    const int rows = g.B * g.R;
+    t.NB = g.C >= 8 ? kBins : (g.C >= 4 ? 512 : (g.C >= 2 ? 256 : 128));
+    t.HC = std::max(1, std::min(16, g.C / 5));
+    t.KC = std::max(1, std::min(std::min(64, g.C), (1024 + rows - 1) / rows));
+    const uint32_t bytes = (uint32_t)((uint64_t)g.C * kRowArea - sizeof(RowCut));
+    t.bins_off = (uint32_t)(g.C * sizeof(Moments));
+    t.cnt_off = t.bins_off + (uint32_t)(t.HC * t.NB * 8);
+    t.cand_off = t.cnt_off + (uint32_t)(t.KC * 4 * 4);
+    // (segments fill unevenly: twice the list's room where there is space)
+    t.seg = std::min((int)((bytes - t.cand_off) / sizeof(Member)), 2 * kCandMost) / (t.KC * 4);
+    return t;
+}
+
 }  // namespace
 
 uint64_t accept_scratch_bytes(const yuuka_accept_params &p) {
     const Geo g = make_geo(p);
     const uint64_t n = (uint64_t)g.B * g.R * g.C;
     return ((n * sizeof(Stat) + 255) & ~255ull) + n * sizeof(double) +
-           (uint64_t)g.B * g.R * (sizeof(double) + sizeof(Cut)) + 256 + n * sizeof(Hist0);
+           (uint64_t)g.B * g.R * (sizeof(double) + sizeof(Cut)) + 256 + n * kRowArea;
 }
 
 hipError_t launch_router_normal(float *logits, int rows, int E, uint64_t seed, uint32_t layer, const uint64_t *step,
@@ -1010,11 +1619,9 @@ hipError_t launch_verify_accept(const float *logits, const int32_t *drafts, int3
     Stat *stats = reinterpret_cast<Stat *>(base);
     double *sums = reinterpret_cast<double *>(base + ((n * sizeof(Stat) + 255) & ~255ull));
     double *wdraft = sums + n;
-    Cut *cuts = reinterpret_cast<Cut *>(wdraft + (uint64_t)g.B * g.R);
-    Hist0 *h0 = reinterpret_cast<Hist0 *>(
-        (reinterpret_cast<uintptr_t>(cuts + (uint64_t)g.B * g.R) + 255) & ~(uintptr_t)255);
     const bool stochastic = p.mode == YUUKA_ACCEPT_STOCHASTIC && p.temperature > 0.0f && p.top_k != 1;
-    const double t = stochastic ? (double)p.temperature : 1.0;
+    const double td = stochastic ? std::min((double)p.temperature, 1e300) : 1.0;
+    const Temp t{td, 1.0 / td};
     // top_p 0 means off (sampling.go:46-48); top_k at or above the vocabulary keeps everything.
     const bool top_k_on = p.top_k > 1 && p.top_k < p.vocab;
     const bool top_p_on = p.top_p > 0.0f && p.top_p < 1.0f;
@@ -1025,32 +1632,53 @@ hipError_t launch_verify_accept(const float *logits, const int32_t *drafts, int3
     // one wave per chunk up to 8 logits per lane, else a workgroup per chunk
     const int wpc = g.L <= 512 * 4 ? 1 : 4;
     const dim3 sgrid((unsigned)((g.C + 4 / wpc - 1) / (4 / wpc)), (unsigned)g.R, (unsigned)g.B);
-    accept_stats_kernel<<<sgrid, 256, 0, stream>>>(logits, g, stats, vec, wpc);
-    const dim3 sel((unsigned)g.R, (unsigned)g.B);
-    const int tk = top_k_on ? (int)p.top_k : 0;
-    if (truncate && !top_p_on) {
-        accept_select_kernel<<<sel, kSelWaves * 64, 0, stream>>>(logits, g, stats, tk, 1.0f, t, cuts, 0, nullptr);
-    } else if (truncate) {
-        // top-k cut, then the first top-p digit over all chunks in parallel,
-        // then the remaining top-p digits per row
-        if (top_k_on)
-            accept_select_kernel<<<sel, kSelWaves * 64, 0, stream>>>(logits, g, stats, tk, 1.0f, t, cuts, 1, nullptr);
-        accept_hist_kernel<<<grid, 256, 0, stream>>>(logits, g, stats, top_k_on ? cuts : nullptr, t, h0);
-        static bool attr = false;
-        constexpr uint32_t cand_lds = kCandCap * 4 + kSelWaves * 4;
-        if (!attr) {
-            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(accept_select_kernel),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)cand_lds);
-            attr = true;
-        }
-        accept_select_kernel<<<sel, kSelWaves * 64, cand_lds, stream>>>(logits, g, stats, tk, p.top_p, t, cuts, 2, h0);
+    if (!truncate) {
+        accept_stats_kernel<false><<<sgrid, 256, 0, stream>>>(logits, g, stats, vec, wpc, nullptr);
+        if (stochastic) accept_weights_kernel<<<grid, 256, 0, stream>>>(logits, g, drafts, stats, t, sums, wdraft);
+        accept_finalize_kernel<<<(unsigned)g.B, 256, 0, stream>>>(logits, g, drafts, stats, sums, wdraft,
+                                                                 stochastic ? 1 : 0, t, p.seed, p.step, p.request_base,
+                                                                 result, debug, step_dev, forced);
+        return hipGetLastError();
     }
-    const Cut *cut_arg = truncate ? cuts : nullptr;
-    if (stochastic)
-        accept_weights_kernel<<<grid, 256, 0, stream>>>(logits, g, drafts, stats, cut_arg, t, sums, wdraft);
-    accept_finalize_kernel<<<(unsigned)g.B, 256, 0, stream>>>(logits, g, drafts, stats, sums, wdraft, cut_arg,
-                                                             stochastic ? 1 : 0, t, p.seed, p.step,
-                                                             p.request_base, result, debug, step_dev, forced);
+    uint8_t *area = reinterpret_cast<uint8_t *>((reinterpret_cast<uintptr_t>(wdraft + (uint64_t)g.B * g.R) + 255) &
+                                                ~(uintptr_t)255);
+    const TruncGeo tg = trunc_geo(g);
+    const int tk = top_k_on ? (int)p.top_k : 0;
+    const float tp = top_p_on ? p.top_p : 1.0f;
+    const dim3 rgrid((unsigned)g.R, (unsigned)g.B);
+    const dim3 hgrid((unsigned)tg.HC, (unsigned)g.R, (unsigned)g.B), kgrid((unsigned)tg.KC, (unsigned)g.R, (unsigned)g.B);
+    const uint32_t bins_lds = (uint32_t)(kBinWaves * tg.NB) * (top_k_on ? 4u : 8u);
+    static bool attr = false;
+    if (!attr) {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(accept_cut_kernel),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, kCandMost * (int)sizeof(Member));
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(accept_bins_kernel<false>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, kBinWaves * kBins * 8);
+        attr = true;
+    }
+    int cand = std::min(kCandMost, tg.KC * 4 * tg.seg);
+    const int direct = (int)p.vocab <= kDirectMost ? 1 : 0;
+    if (direct) {
+        accept_stats_kernel<false><<<sgrid, 256, 0, stream>>>(logits, g, stats, vec, wpc, nullptr);
+        cand = g.V;
+    } else if (top_k_on) {
+        accept_stats_kernel<true><<<sgrid, 256, 0, stream>>>(logits, g, stats, vec, wpc, area);
+        accept_bins_kernel<true><<<hgrid, 64 * kBinWaves, bins_lds, stream>>>(logits, g, tg, drafts, stats, t, area);
+        accept_collect_kernel<true><<<kgrid, 256, 0, stream>>>(logits, g, tg, drafts, stats, tk, tp, t, area);
+    } else {
+        accept_stats_kernel<true><<<sgrid, 256, 0, stream>>>(logits, g, stats, vec, wpc, area);
+        accept_bins_kernel<false><<<hgrid, 64 * kBinWaves, bins_lds, stream>>>(logits, g, tg, drafts, stats, t, area);
+        accept_collect_kernel<false><<<kgrid, 256, 0, stream>>>(logits, g, tg, drafts, stats, tk, tp, t, area);
+    }
+    accept_cut_kernel<<<rgrid, 64 * kSelWaves, (uint32_t)cand * sizeof(Member), stream>>>(logits, g, tg, drafts, stats, tk,
+                                                                                         tp, t, area, direct);
+    // chunks of the drawn row: at most 64 (one per lane of pick), and their
+    // sums fit the per-chunk sums' place
+    const int RC = std::min(64, g.R * g.C);
+    accept_resample_kernel<<<dim3((unsigned)RC, (unsigned)g.B), 256, 0, stream>>>(
+        logits, g, RC, drafts, area, t, p.seed, p.step, p.request_base, step_dev, forced, sums);
+    accept_pick_kernel<<<(unsigned)g.B, 256, 0, stream>>>(logits, g, RC, drafts, area, sums, t, p.seed, p.step,
+                                                         p.request_base, step_dev, forced, result, debug);
     return hipGetLastError();
 }
 

@@ -227,6 +227,66 @@ def test_fused_gemm_many_rows(dev, stream, segs, k, rows, norm):
         _check(gv, _want(dt, w, n, k, y), budget=MANY_BUDGET)
 
 
+# Row counts at the edges of one, two and three row tiles and past them, odd
+# super-block counts (1: two of the four K parts are empty; 3, 5: unequal
+# parts), channel counts off the tiles of 16 and of 8 + 8, both launches of the
+# few-row kernel (with and without K splits) and a segment of one channel.
+FEW = [
+    ([(O.Q6_K, 1)], 256, 9, True),
+    ([(O.Q4_K, 33), (O.Q6_K, 17), (O.Q4_K, 1)], 256, 16, False),
+    ([(O.Q4_K, 1000), (O.Q6_K, 9000)], 768, 16, True),   # more channels than CUs x 32
+    ([(O.Q6_K, 8209), (O.Q4_K, 31)], 1280, 17, False),
+    ([(O.Q4_K, 530)], 3328, 32, True),
+    ([(O.Q6_K, 47), (O.Q4_K, 8200)], 512, 33, False),
+    ([(O.Q4_K, 100), (O.Q6_K, 100)], 2816, 48, True),
+    ([(O.Q6_K, 100), (O.Q4_K, 100)], 2816, 49, True),
+    ([(O.Q6_K, 70)], 4352, 32, False),                   # long K: few rows up to 32,
+    ([(O.Q6_K, 70)], 4352, 33, False),                   # staged from 33
+    ([(O.Q4_K, 24580)], 256, 17, True),                  # past the few-row kernel's channels
+]
+
+
+def _rounding_bound(dt, w, n, k, y):
+    """Activations round by at most 2^-11 of themselves, Q6_K weights too: no
+    output is off by more than 2^-10 of sum |y| |w|, at most |y| |w|
+    (Cauchy-Schwarz)."""
+    wn = np.linalg.norm(O.dequantize(dt, w, n, k).astype(np.float64), axis=1)
+    return 2.0 ** -10 * np.linalg.norm(y.astype(np.float64), axis=1)[:, None] * wn[None, :]
+
+
+@pytest.mark.parametrize("segs,k,rows,norm", FEW)
+def test_fused_gemm_few_row_edges(dev, stream, segs, k, rows, norm):
+    rng = np.random.default_rng(k * 5 + rows + len(segs))
+    x = rng.normal(0, 1, (rows, k)).astype(np.float32)
+    x[rows // 2] = 0.0                       # a row without values
+    x[0, : k // 2] *= 1e-4                   # super-blocks of different scale
+    g = rng.normal(1, 0.1, k).astype(np.float32) if norm else None
+    ws = [synth.quant_matrix(rng, dt, n, k) for dt, n in segs]
+    got = _run(dev, stream, x, [(dt, w, n) for (dt, n), w in zip(segs, ws)], k, rows, norm=g)
+    y = O.rmsnorm_rows(x, g, 1e-6) if norm else x
+    for (dt, n), w, gv in zip(segs, ws, got):
+        want = _want(dt, w, n, k, y).astype(np.float64)
+        bound = _rounding_bound(dt, w, n, k, y)
+        assert np.all(np.abs(gv - want) <= bound + 1e-30)
+        assert np.all(gv[rows // 2] == 0.0)
+
+
+@pytest.mark.parametrize("n,k,rows", [(7, 256, 9), (2049, 768, 16), (2560, 2560, 30), (5001, 512, 48)])
+def test_fused_gemm_few_row_swiglu_edges(dev, stream, n, k, rows):
+    rng = np.random.default_rng(n + k + rows)
+    x = rng.normal(0, 1, (rows, k)).astype(np.float32)
+    g = rng.normal(1, 0.1, k).astype(np.float32)
+    wg, wu = synth.quant_matrix(rng, O.Q4_K, n, k), synth.quant_matrix(rng, O.Q4_K, n, k)
+    got = _run(dev, stream, x, [(O.Q4_K, wg, n), (O.Q4_K, wu, n)], k, rows, hip.EPI_SWIGLU, norm=g)[0]
+    y = O.rmsnorm_rows(x, g, 1e-6)
+    gate, up = (_want(O.Q4_K, w, n, k, y).astype(np.float64) for w in (wg, wu))
+    silu = gate / (1 + np.exp(-np.clip(gate, -700, 700)))
+    # either product's rounding as above, through SiLU (slope at most 1.1) and
+    # the product
+    eg, eu = (_rounding_bound(O.Q4_K, w, n, k, y) for w in (wg, wu))
+    assert np.all(np.abs(got - silu * up) <= 1.1 * eg * np.abs(up) + np.abs(silu) * eu + 1.1 * eg * eu + 1e-30)
+
+
 def test_fused_gemm_many_rows_epilogues(dev, stream):
     """SwiGLU, residual, output maps and the gated head norm at 37 rows."""
     rng = np.random.default_rng(31)

@@ -7,7 +7,9 @@
 // At a few rows the fused streaming kernel reads every weight once per
 // launch; a batch of B requests x (k+1) rows would read them once per 8-row
 // block. Here each weight super-block is read once per block of 48 rows (80
-// for 49..80 rows), and the products run on v_mfma_f32_16x16x32_f16:
+// for 49..80 rows), and the products run on v_mfma_f32_16x16x32_f16 (this
+// describes bg_gemm_kernel; up to 48 rows of moderate width take
+// bg_few_kernel, the same products from registers, see there):
 //
 //  * prologue (one workgroup per row and group of 8 super-blocks): y =
 //    prologue(x) computed as the reference computes it (recurrent.go:39-50
@@ -73,6 +75,10 @@ constexpr float kBgRange = 256.0f;  // |y / scale| <= kBgRange
 //   h      [sb][tile][sub-block j][group g][row c][8 FP16]  (8 KB per tile)
 //   sums   [sb][tile][row c][16 FP16]                       (512 B per tile)
 //   scales [sb][tile * 16 + c] float
+// Within each four elements of K the order is 0, 2, 1, 3, the order in which
+// the 16-bit halves of a weight word and of the word shifted by a byte give
+// its quants as FP16 pairs (the product sums over K, so any order is exact
+// that both operands follow).
 //   ss     [row][kBgSsGroups] float64 sums of squares of x over the
 //          prologue workgroups' super-block groups (RMSNorm prologues: the
 //          GEMM applies the row's 1/rms to its sums)
@@ -343,7 +349,7 @@ __global__ __launch_bounds__(kPrThreads) void bg_prologue_kernel(const FusedGemm
         const float inv = m > 0.f ? kBgRange / m : 0.f;
         const _Float16 h0 = (_Float16)(y.x * inv), h1 = (_Float16)(y.y * inv), h2 = (_Float16)(y.z * inv),
                        h3 = (_Float16)(y.w * inv);
-        *reinterpret_cast<uint2 *>(h_at(sb)) = make_uint2(h2bits(h0, h1), h2bits(h2, h3));
+        *reinterpret_cast<uint2 *>(h_at(sb)) = make_uint2(h2bits(h0, h2), h2bits(h1, h3));
         // sub-block lane >> 3: eight lanes of four values
         const float s = group8_sum(((float)h0 + (float)h1) + ((float)h2 + (float)h3));
         if ((lane & 7) == 0) {
@@ -447,7 +453,7 @@ __device__ __forceinline__ float out_map(const FusedSeg &S, int n, float v) {
     }
 }
 
-// FP16 pairs from byte pairs: (x & mask) | 0x6400 in each 16-bit half is
+// FP16 pairs from the halves of a word: (x & mask) | 0x6400 in each 16-bit half is
 // 1024 + x as FP16 (x < 1024).
 __device__ __forceinline__ half2v magic_pair(uint32_t w, uint32_t mask) {
     uint32_t r;  // one v_and_or_b32 (written out: the compiler splits it when the and is shared)
@@ -543,19 +549,17 @@ __device__ __forceinline__ void bg_super_q4(const WQ4 &cur, const uint8_t *st, f
         // nibbles 2 jp + 1. Low: (1024 + q) sc - 1024 sc; high, masked in
         // place: (1024 + 16 q) (sc / 16) - 64 sc. Both are q sc exactly (one
         // rounding of an exact value below 2048).
-        const uint32_t w0 = (uint32_t)cur.q[jp], w1 = (uint32_t)(cur.q[jp] >> 32);
-        const uint32_t p01 = __builtin_amdgcn_perm(0u, w0, 0x0c010c00u), p23 = __builtin_amdgcn_perm(0u, w0, 0x0c030c02u);
-        const uint32_t p45 = __builtin_amdgcn_perm(0u, w1, 0x0c010c00u), p67 = __builtin_amdgcn_perm(0u, w1, 0x0c030c02u);
+        const uint32_t w0 = (uint32_t)cur.q[jp], w1 = (uint32_t)(cur.q[jp] >> 32), v0 = w0 >> 8, v1 = w1 >> 8;
         const half2v se = splat_h((float)sce), so = splat_h(0.0625f * (float)sco);
         const half2v ce = splat_h(-1024.f * (float)sce), co = splat_h(-64.f * (float)sco);
-        const half8 be = pack8(__builtin_elementwise_fma(magic_pair(p01, 0x000F000Fu), se, ce),
-                               __builtin_elementwise_fma(magic_pair(p23, 0x000F000Fu), se, ce),
-                               __builtin_elementwise_fma(magic_pair(p45, 0x000F000Fu), se, ce),
-                               __builtin_elementwise_fma(magic_pair(p67, 0x000F000Fu), se, ce));
-        const half8 bo = pack8(__builtin_elementwise_fma(magic_pair(p01, 0x00F000F0u), so, co),
-                               __builtin_elementwise_fma(magic_pair(p23, 0x00F000F0u), so, co),
-                               __builtin_elementwise_fma(magic_pair(p45, 0x00F000F0u), so, co),
-                               __builtin_elementwise_fma(magic_pair(p67, 0x00F000F0u), so, co));
+        const half8 be = pack8(__builtin_elementwise_fma(magic_pair(w0, 0x000F000Fu), se, ce),
+                               __builtin_elementwise_fma(magic_pair(v0, 0x000F000Fu), se, ce),
+                               __builtin_elementwise_fma(magic_pair(w1, 0x000F000Fu), se, ce),
+                               __builtin_elementwise_fma(magic_pair(v1, 0x000F000Fu), se, ce));
+        const half8 bo = pack8(__builtin_elementwise_fma(magic_pair(w0, 0x00F000F0u), so, co),
+                               __builtin_elementwise_fma(magic_pair(v0, 0x00F000F0u), so, co),
+                               __builtin_elementwise_fma(magic_pair(w1, 0x00F000F0u), so, co),
+                               __builtin_elementwise_fma(magic_pair(v1, 0x00F000F0u), so, co));
 #pragma unroll
         for (int t = 0; t < NT; t++) {
             const half8 ae = *reinterpret_cast<const half8 *>(la + t * 8192 + (2 * jp) * 1024);
@@ -603,8 +607,7 @@ __device__ __forceinline__ void bg_super_q6(const WQ6 &cur, const uint8_t *st, f
         auto one = [&](uint32_t pq) __attribute__((always_inline)) {
             return (magic_pair(pq, 0x003F003Fu) + off) * s2;  // (1024 + q + 32) - 1056 = q, times sc
         };
-        const half8 bj = pack8(one(__builtin_amdgcn_perm(0u, w0, 0x0c010c00u)), one(__builtin_amdgcn_perm(0u, w0, 0x0c030c02u)),
-                               one(__builtin_amdgcn_perm(0u, w1, 0x0c010c00u)), one(__builtin_amdgcn_perm(0u, w1, 0x0c030c02u)));
+        const half8 bj = pack8(one(w0), one(w0 >> 8), one(w1), one(w1 >> 8));
 #pragma unroll
         for (int t = 0; t < NT; t++)
             acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const half8 *>(la + t * 8192 + j * 1024), bj,
@@ -684,6 +687,22 @@ __device__ __forceinline__ void bg_main(const BgArgs &A, uint8_t *lds, int T0, b
     }
 }
 
+// RMSNorm prologue: a row's 1 / rms from the prologue's group sums, added in
+// group order (forward.go:460-470).
+__device__ __forceinline__ float bg_row_inv(const BgArgs &A, int row) {
+    const int G = (A.f.K / 256 + kPrWaves - 1) / kPrWaves;
+    const double *ps = A.q.ss + (uint64_t)row * kBgSsGroups;
+    double v[kBgSsGroups];
+#pragma unroll
+    for (int gi = 0; gi < kBgSsGroups; gi++) v[gi] = ps[min(gi, G - 1)];
+    double t = 0.0;
+#pragma unroll
+    for (int gi = 0; gi < kBgSsGroups; gi++)
+        if (gi < G) t += v[gi];
+    const float mean = (float)(t / (double)A.f.K);
+    return (float)(1.0 / sqrt((double)(mean + A.f.eps)));
+}
+
 template <int NT>
 __global__ __launch_bounds__(kBgThreads) __attribute__((amdgpu_waves_per_eu(NT > 4 ? 2 : 4))) void bg_gemm_kernel(
     const BgArgs A) {
@@ -717,24 +736,13 @@ __global__ __launch_bounds__(kBgThreads) __attribute__((amdgpu_waves_per_eu(NT >
     for (int t = 0; t < NT; t++)
 #pragma unroll
         for (int i = 0; i < 4; i++) y[t][i] = 0.f;
-    // RMSNorm prologue: the 1 / rms of the block's rows from the prologue's
-    // group sums (added in group order; forward.go:460-470), published by
-    // the main loop's first barrier
+    // RMSNorm prologue: the 1 / rms of the block's rows, published by the
+    // main loop's first barrier
     __shared__ float row_inv[kRowsB];
     const bool rnorm = F.norm != nullptr && F.gate == nullptr;
     auto pre = [&]() __attribute__((always_inline)) {
         if (!rnorm || threadIdx.x >= kRowsB) return;
-        const int row = min(m0 + (int)threadIdx.x, F.rows - 1), G = (F.K / 256 + kPrWaves - 1) / kPrWaves;
-        const double *ps = A.q.ss + (uint64_t)row * kBgSsGroups;
-        double v[kBgSsGroups];
-#pragma unroll
-        for (int gi = 0; gi < kBgSsGroups; gi++) v[gi] = ps[min(gi, G - 1)];
-        double t = 0.0;
-#pragma unroll
-        for (int gi = 0; gi < kBgSsGroups; gi++)
-            if (gi < G) t += v[gi];
-        const float mean = (float)(t / (double)F.K);
-        row_inv[threadIdx.x] = (float)(1.0 / sqrt((double)(mean + F.eps)));
+        row_inv[threadIdx.x] = bg_row_inv(A, min(m0 + (int)threadIdx.x, F.rows - 1));
     };
     if (S.dtype == kQ6K) bg_main<kQ6K, NT>(A, lds, m0 / 16, live, wrow, y, pre);
     else bg_main<kQ4K, NT>(A, lds, m0 / 16, live, wrow, y, pre);
@@ -797,6 +805,299 @@ __global__ __launch_bounds__(kBgThreads) __attribute__((amdgpu_waves_per_eu(NT >
         }
 }
 
+// ------------------------------------------------- GEMM of up to 48 rows
+// At few row tiles an operand that is staged through LDS is read back for one
+// to three MFMAs only, and the stages' barriers leave the loads of one stage
+// in flight. Here the operands stay in registers and the waves are
+// independent: a wave owns TW tiles of 16 channels (which share its A
+// operands, read straight from L2 in operand order), NR row tiles and every
+// fourth half super-block of the workgroup's K range; the four parts of a
+// tile are added through LDS at the end, in order. The loads of the A
+// operands bound it as much as those of the weights (in a trial over 16 rows
+// of 2560 -> 151936 Q6_K, 134 us with one channel tile to a wave took 97
+// without the A loads and 100 with the weights' from one place).
+//
+// Half a super-block (sub-blocks 4 h .. 4 h + 3) of one channel, as lane
+// (c, g) needs it.
+struct Win {  // 12 bytes from the dword at or below an even address
+    uint32_t w[3];
+};
+struct HQ4 {
+    uint4 hdr;      // d, dmin, 12 scale bytes
+    uint64_t q[2];  // bytes [16 + 64 h + 32 p + 8 g, +8)
+};
+struct HQ6 {
+    Win ql[2];   // ql bytes [64 h + 32 p + 8 g, +8)
+    Win qh;      // qh bytes [32 h + 8 g, +8)
+    Win sc;      // int8 scales 8 h .. 8 h + 7
+    uint16_t d;
+};
+__device__ __forceinline__ void load_win(Win &v, const uint8_t *p) {
+    const uint32_t sh = (uint32_t)reinterpret_cast<uintptr_t>(p) & 3;
+    const uint32_t *w = reinterpret_cast<const uint32_t *>(p - sh);  // pointer arithmetic keeps the global address space
+#pragma unroll
+    for (int i = 0; i < 3; i++) v.w[i] = w[i];
+}
+__device__ __forceinline__ uint64_t win8(const Win &v, uint32_t sh) {
+    return (uint64_t)__builtin_amdgcn_alignbyte(v.w[1], v.w[0], sh) |
+           ((uint64_t)__builtin_amdgcn_alignbyte(v.w[2], v.w[1], sh) << 32);
+}
+__device__ __forceinline__ void load_half(HQ4 &w, const uint8_t *blk, int h, int g) {
+    w.hdr = *reinterpret_cast<const uint4 *>(blk);
+#pragma unroll
+    for (int p = 0; p < 2; p++) w.q[p] = *reinterpret_cast<const uint64_t *>(blk + 16 + 64 * h + 32 * p + 8 * g);
+}
+__device__ __forceinline__ void load_half(HQ6 &w, const uint8_t *blk, int h, int g) {
+#pragma unroll
+    for (int p = 0; p < 2; p++) load_win(w.ql[p], blk + 64 * h + 32 * p + 8 * g);
+    load_win(w.qh, blk + 128 + 32 * h + 8 * g);
+    // (from byte 192 or 198: nothing past byte 210 is read)
+    load_win(w.sc, blk + 192 + 6 * h);
+    w.d = *reinterpret_cast<const uint16_t *>(blk + 208);
+}
+
+// Two 6-bit values of a word's bytes I and I + 1 as FP16.
+template <int I> __device__ __forceinline__ half2v pair6(uint32_t w) {
+    const uint32_t v = __builtin_amdgcn_perm(0u, w, I == 0 ? 0x0c010c00u : 0x0c030c02u) | 0x64006400u;
+    return __builtin_bit_cast(half2v, v) - half2v{(_Float16)1024.f, (_Float16)1024.f};
+}
+
+// B operands sc q of the half's four sub-blocks and (first half) the mins;
+// the same values as bg_super_q4 and bg_super_q6 build.
+__device__ __forceinline__ void half_operands(const HQ4 &w, int h, int g, uint32_t, half8 (&b)[4], half8 &mins) {
+    const uint32_t q0 = w.hdr.y, q1 = w.hdr.z, q2 = w.hdr.w;
+    // tensor/quant.go:96-103 getScaleMinK4, four sub-blocks to a word
+    const uint32_t sc_lo = q0 & 0x3f3f3f3fu, sc_hi = (q2 & 0x0f0f0f0fu) | ((q0 >> 2) & 0x30303030u);
+    const uint32_t sc = h ? sc_hi : sc_lo;
+#pragma unroll
+    for (int p = 0; p < 2; p++) {
+        const half2v sp = p ? pair6<2>(sc) : pair6<0>(sc);  // of the low and the high nibbles
+        const half2v mul = sp * half2v{(_Float16)1.f, (_Float16)0.0625f};
+        const half2v off = sp * half2v{(_Float16)-1024.f, (_Float16)-64.f};
+        const half2v se{mul[0], mul[0]}, ce{off[0], off[0]}, so{mul[1], mul[1]}, co{off[1], off[1]};
+        const uint32_t w0 = (uint32_t)w.q[p], w1 = (uint32_t)(w.q[p] >> 32), v0 = w0 >> 8, v1 = w1 >> 8;
+        b[2 * p] = pack8(__builtin_elementwise_fma(magic_pair(w0, 0x000F000Fu), se, ce),
+                         __builtin_elementwise_fma(magic_pair(v0, 0x000F000Fu), se, ce),
+                         __builtin_elementwise_fma(magic_pair(w1, 0x000F000Fu), se, ce),
+                         __builtin_elementwise_fma(magic_pair(v1, 0x000F000Fu), se, ce));
+        b[2 * p + 1] = pack8(__builtin_elementwise_fma(magic_pair(w0, 0x00F000F0u), so, co),
+                             __builtin_elementwise_fma(magic_pair(v0, 0x00F000F0u), so, co),
+                             __builtin_elementwise_fma(magic_pair(w1, 0x00F000F0u), so, co),
+                             __builtin_elementwise_fma(magic_pair(v1, 0x00F000F0u), so, co));
+    }
+    if (h == 0) {  // K slots 0..15 (g < 2) hold the mins, the others zero
+        const uint32_t mlo = q1 & 0x3f3f3f3fu, mhi = ((q2 >> 4) & 0x0f0f0f0fu) | ((q1 >> 2) & 0x30303030u);
+        mins = g < 2 ? pack8(pair6<0>(mlo), pair6<2>(mlo), pair6<0>(mhi), pair6<2>(mhi)) : half8{};
+    }
+}
+__device__ __forceinline__ void half_operands(const HQ6 &w, int h, int g, uint32_t sh, half8 (&b)[4], half8 &) {
+    const uint64_t l0 = win8(w.ql[0], sh), l1 = win8(w.ql[1], sh), hh = win8(w.qh, sh);
+    // the eight scales: the second half's may start 4 bytes into the window
+    const bool far = h && sh == 0;
+    const uint32_t slo = far ? w.sc.w[1] : __builtin_amdgcn_alignbyte(w.sc.w[1], w.sc.w[0], sh);
+    const uint32_t shi = far ? w.sc.w[2] : __builtin_amdgcn_alignbyte(w.sc.w[2], w.sc.w[1], sh);
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        // u = q + 32 at bits 4..9 of 0x5400 is 64 + u as FP16: the four low
+        // bits of the even (odd) bytes of a word moved to 4..7, the two high
+        // bits to 8..9; then (64 + u) sc - 96 sc, one rounding of q sc
+        const _Float16 sc = (_Float16)(int16_t)(int8_t)((q < 2 ? slo : shi) >> (16 * (q & 1) + 8 * (g >> 1)));
+        const half2v s2{sc, sc}, off = s2 * half2v{(_Float16)-96.f, (_Float16)-96.f};
+        auto one = [&](uint32_t l, uint32_t hi, int odd) __attribute__((always_inline)) {
+            const int ls = 4 * (q >> 1) + 8 * odd - 4, hs = 2 * q + 8 * odd - 8;  // right shifts
+            const uint32_t lw = ls < 0 ? l << -ls : l >> ls, hw = hs < 0 ? hi << -hs : hi >> hs;
+            uint32_t r;
+            asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(lw), "v"(0x00F000F0u), "v"(0x54005400u));
+            asm("v_and_or_b32 %0, %1, %2, %0" : "+v"(r) : "v"(hw), "v"(0x03000300u));
+            return __builtin_elementwise_fma(__builtin_bit_cast(half2v, r), s2, off);
+        };
+        const uint64_t l = q & 1 ? l1 : l0;
+        const uint32_t w0 = (uint32_t)l, w1 = (uint32_t)(l >> 32), h0 = (uint32_t)hh, h1 = (uint32_t)(hh >> 32);
+        b[q] = pack8(one(w0, h0, 0), one(w0, h0, 1), one(w1, h1, 0), one(w1, h1, 1));
+    }
+}
+
+// One wave's part kw of the tiles [tile, tile + TW) of segment seg (SwiGLU: 8
+// gate channels and the same 8 of up to a tile) over the super-blocks [sb_lo,
+// sb_lo + n). Every load is issued, its index clamped. `pre` runs behind the
+// first loads.
+template <int DT, int NR, int TW, class Pre>
+__device__ __forceinline__ void bg_few(const BgArgs &A, int seg, int tile, int sb_lo, int n, int kw,
+                                       f32x4 (&y)[NR][TW], Pre pre) {
+    typedef typename std::conditional<DT == kQ4K, HQ4, HQ6>::type Raw;
+    constexpr int blk = DT == kQ4K ? 144 : 210;
+    const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4, h = kw & 1;
+    // the wave's half super-blocks: half h of super-blocks kw / 2, kw / 2 + 2, ...
+    const int nu = (2 * n - kw + 3) / 4;
+    if (nu <= 0) {  // uniform
+        pre();
+        return;
+    }
+    const FusedSeg &sg = A.f.seg[seg];
+    const uint8_t *w = static_cast<const uint8_t *>(A.swiglu && c >= 8 ? A.f.seg[1].w : sg.w);
+    const uint8_t *wrow[TW];
+#pragma unroll
+    for (int t = 0; t < TW; t++) {
+        const int ch = A.swiglu ? (tile + t) * 8 + (c & 7) : (tile + t) * 16 + c;
+        wrow[t] = w + (uint64_t)min(ch, sg.n - 1) * sg.row_bytes + (uint64_t)sb_lo * blk;
+    }
+    const int tiles = bg_rows16(A.f.rows) / 16;
+    int rt[NR];
+#pragma unroll
+    for (int r = 0; r < NR; r++) rt[r] = min(r, tiles - 1);
+    auto at = [&](int i) __attribute__((always_inline)) { return (kw >> 1) + 2 * min(i, nu - 1); };
+    Raw raw[2][TW];
+    half8 a[4][NR], as[NR];
+    float4 xs[NR];
+    auto load = [&](int slot, int t, int i) __attribute__((always_inline)) {
+        load_half(raw[slot][t], wrow[t] + (uint32_t)(at(i) * blk), h, g);
+    };
+    auto load_a = [&](int j, int i) __attribute__((always_inline)) {
+        const uint64_t sb = (uint64_t)(sb_lo + at(i)) * tiles;
+#pragma unroll
+        for (int r = 0; r < NR; r++)
+            a[j][r] = *reinterpret_cast<const half8 *>(reinterpret_cast<const uint8_t *>(A.q.h) + (sb + rt[r]) * 8192 +
+                                                       (4 * h + j) * 1024 + (uint32_t)lane * 16);
+    };
+    auto load_s = [&](int i) __attribute__((always_inline)) {
+        const uint64_t sb = (uint64_t)(sb_lo + at(i)) * tiles;
+#pragma unroll
+        for (int r = 0; r < NR; r++) {
+            xs[r] = *reinterpret_cast<const float4 *>(A.q.scales + (sb + rt[r]) * 16 + 4 * g);
+            if (DT == kQ4K)
+                as[r] = *reinterpret_cast<const half8 *>(reinterpret_cast<const uint8_t *>(A.q.sums) + (sb + rt[r]) * 512 +
+                                                         (uint32_t)(c * 32 + (g & 1) * 16));
+        }
+    };
+    auto step = [&](int slot, int i) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < TW; t++) {
+            half8 b[4], bm;
+            const uint32_t sh = (uint32_t)(reinterpret_cast<uintptr_t>(wrow[t]) + (uint32_t)(at(i) * blk)) & 3;
+            half_operands(raw[slot][t], h, g, sh, b, bm);
+            float d, dmin = 0.f;
+            if constexpr (DT == kQ4K) {
+                d = h2f((uint16_t)(raw[slot][t].hdr.x & 0xffffu));
+                dmin = h2f((uint16_t)(raw[slot][t].hdr.x >> 16));
+            } else {
+                d = h2f(raw[slot][t].d);
+            }
+            f32x4 acc[NR];
+#pragma unroll
+            for (int r = 0; r < NR; r++) acc[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+#pragma unroll
+                for (int r = 0; r < NR; r++)
+                    acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[j][r], b[j], acc[r], 0, 0, 0);
+                if (t == TW - 1) load_a(j, i + 1);
+            }
+            if (DT == kQ4K && h == 0) {
+#pragma unroll
+                for (int r = 0; r < NR; r++) {
+                    const f32x4 mn = __builtin_amdgcn_mfma_f32_16x16x32_f16(as[r], bm, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                    y[r][t] += f32x4{xs[r].x, xs[r].y, xs[r].z, xs[r].w} * (d * acc[r] - dmin * mn);
+                }
+            } else {
+#pragma unroll
+                for (int r = 0; r < NR; r++) y[r][t] += f32x4{xs[r].x, xs[r].y, xs[r].z, xs[r].w} * (d * acc[r]);
+            }
+        }
+        load_s(i + 1);
+        // (last, so that a wait for the next step's A operands leaves them in flight)
+#pragma unroll
+        for (int t = 0; t < TW; t++) load(slot, t, i + 2);
+    };
+#pragma unroll
+    for (int t = 0; t < TW; t++) load(0, t, 0);
+#pragma unroll
+    for (int j = 0; j < 4; j++) load_a(j, 0);
+    load_s(0);
+#pragma unroll
+    for (int t = 0; t < TW; t++) load(1, t, 1);
+    pre();
+    int i = 0;
+#pragma unroll 1
+    for (; i + 2 <= nu; i += 2) {
+        step(0, i);
+        step(1, i + 1);
+    }
+    if (i < nu) step(0, i);
+}
+
+constexpr int kFewThreads = 256;
+template <int NR, int TW>
+__global__ __launch_bounds__(kFewThreads, NR == 1 ? 3 : 2) void bg_few_kernel(const BgArgs A) {
+    __shared__ f32x4 sums[4][TW][NR][64];
+    __shared__ float row_inv[16 * NR];
+    const FusedGemmArgs &F = A.f;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int c = lane & 15, g = lane >> 4;
+    const int nsb = F.K / 256;
+    const int sb_lo = (int)((int64_t)nsb * blockIdx.z / A.splits);
+    const int n = (int)((int64_t)nsb * (blockIdx.z + 1) / A.splits) - sb_lo;
+    const int seg = A.swiglu ? 0 : seg_of(A, blockIdx.x);
+    const int tile0 = ((int)blockIdx.x - A.tiles[seg]) * TW;
+    const FusedSeg &S = F.seg[seg];
+    // RMSNorm prologue: the 1 / rms of the rows, as in bg_gemm_kernel
+    const bool rnorm = F.norm != nullptr && F.gate == nullptr;
+    auto pre = [&]() __attribute__((always_inline)) {
+        if (rnorm && threadIdx.x < 16 * NR) row_inv[threadIdx.x] = bg_row_inv(A, min((int)threadIdx.x, F.rows - 1));
+    };
+    f32x4 y[NR][TW];
+#pragma unroll
+    for (int r = 0; r < NR; r++)
+#pragma unroll
+        for (int t = 0; t < TW; t++) y[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (S.dtype == kQ6K) bg_few<kQ6K, NR, TW>(A, seg, tile0, sb_lo, n, wave, y, pre);
+    else bg_few<kQ4K, NR, TW>(A, seg, tile0, sb_lo, n, wave, y, pre);
+#pragma unroll
+    for (int t = 0; t < TW; t++)
+#pragma unroll
+        for (int r = 0; r < NR; r++) sums[wave][t][r][lane] = y[r][t];
+    __syncthreads();
+    // (one copy of the code: unrolled over the tiles, the float64 exponentials
+    // of the output maps would make it several times as long)
+#pragma unroll 1
+    for (int q = wave; q < NR * TW; q += 4) {
+        const int r = q / TW, t = q % TW, m0 = 16 * r + 4 * g;
+        if (16 * r >= F.rows) break;  // uniform
+        const f32x4 v4 = ((sums[0][t][r][lane] + sums[1][t][r][lane]) + sums[2][t][r][lane]) + sums[3][t][r][lane];
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = rnorm ? __fmul_rn(v4[i], row_inv[m0 + i]) : v4[i];
+        const int ch = A.swiglu ? (tile0 + t) * 8 + (c & 7) : (tile0 + t) * 16 + c;
+        if (A.splits > 1) {  // partial sums of this split; bg_reduce_kernel finishes
+            if (ch >= S.n) continue;
+            const int ncol = A.cols[F.nseg];
+            float *pp = A.part + ((uint64_t)blockIdx.z * F.rows + m0) * ncol + ch +
+                        A.cols[A.swiglu && c >= 8 ? 1 : seg];
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (m0 + i < F.rows) pp[(uint64_t)i * ncol] = v[i];
+        } else if (A.swiglu) {
+            // lanes c and c + 8 hold a channel's gate and up: they swap so
+            // that c finishes rows 0 and 1, c + 8 rows 2 and 3
+            const bool hi = c >= 8;
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const float own = hi ? v[i + 2] : v[i], give = hi ? v[i] : v[i + 2];
+                const float got = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(give), 0x128, 0xf, 0xf, true));
+                const float o = __fmul_rn(silu_ref(hi ? got : own), hi ? own : got);
+                const int m = m0 + i + (hi ? 2 : 0);
+                if (m < F.rows && ch < S.n) S.out[(uint64_t)m * S.n + ch] = o;
+            }
+        } else if (ch < S.n) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                if (m0 + i >= F.rows) continue;
+                const uint64_t o = (uint64_t)(m0 + i) * S.n + ch;
+                S.out[o] = F.epilogue == kEpiResidual ? __fadd_rn(v[i], S.res[o]) : out_map(S, ch, v[i]);
+            }
+        }
+    }
+}
+
 // Sum of the splits in split order, then the epilogue (one thread per output).
 __global__ __launch_bounds__(256) void bg_reduce_kernel(const BgArgs A) {
     const FusedGemmArgs &F = A.f;
@@ -830,12 +1131,26 @@ __global__ __launch_bounds__(256) void bg_reduce_kernel(const BgArgs A) {
     S.out[o] = v;
 }
 
-// Row tiles per workgroup for a launch of `rows` rows (measured at config
-// shapes, prologue + GEMM per launch: 144 rows gate/up 50.1 / 54.7 / 64.2 /
-// 60.7 us at 3 / 4 / 5 / 9 tiles; 68 rows 44.1 / 47.2 / 41.4 / 49.4 us;
-// 40 rows 30.0 / 31.4 / 37.2 / 45.3 us). Five tiles (80 rows, one
-// workgroup per CU) serve 49..80 rows in one block; otherwise blocks of 48
-// rows (three tiles, two workgroups per CU).
+// Launches of up to 48 rows take bg_few_kernel (prologue and GEMM, before ->
+// with it, us: 2560 -> 2 x 9216 SwiGLU at 16 / 30 / 40 rows 29.8 -> 23.0,
+// 31.3 -> 26.5, 32.6 -> 29.6; 2560 -> 6144 + 2048 + 2 x 16 at 16 rows 24.7 ->
+// 19.1; 9216 -> 2560 at 16 / 30 rows 24.0 -> 21.5, 25.0 -> 23.6; 2048 -> 2560
+// at 16 rows 19.9 -> 18.8; 2048 -> 2048 at 40 rows 20.8 -> 18.9), except
+// where the reads of the A operands from L2 outweigh their staging: many
+// channels (40 rows of 2560 -> 60000: 49 us staged, 60 not, Q6_K 65 and 71;
+// 16 rows of 2560 -> 151936 Q6_K: 130 and 139; 40 rows of 2560 -> 40000 Q4_K
+// still 47 and 45.5) and three row tiles over a long K (40 rows of 9216 ->
+// 2560: 25.3 and 26.0).
+constexpr int64_t kFewChannels = 24576;
+bool bg_few_rows(int rows, int K, int64_t channels) {
+    return rows <= (K <= 4096 ? 48 : 32) && channels <= kFewChannels;
+}
+
+// Row tiles per workgroup of bg_gemm_kernel (measured at config shapes,
+// prologue + GEMM per launch: 144 rows gate/up 50.1 / 54.7 / 64.2 / 60.7 us
+// at 3 / 4 / 5 / 9 tiles; 68 rows 44.1 / 47.2 / 41.4 / 49.4 us). Five tiles
+// (80 rows, one workgroup per CU) serve 49..80 rows in one block; otherwise
+// blocks of 48 rows (three tiles, two workgroups per CU).
 int bg_tiles(int rows) { return rows > 48 && rows <= 80 ? 5 : 3; }
 
 template <int NT> const void *bg_kernel_ptr() { return reinterpret_cast<const void *>(bg_gemm_kernel<NT>); }
@@ -857,6 +1172,17 @@ int bg_resident(int nt) {
     return res[nt];
 }
 
+int bg_cus() {
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+            n = 256;
+        return n;
+    }();
+    return cus;
+}
+
 // K splits for a launch of `wgs` workgroups over `nsb` super-blocks: the
 // split count with the least estimated time, in super-block steps,
 //   ceil(wgs * splits / CUs) * (ceil(nsb / splits) + 1) + 0.1 splits,
@@ -868,14 +1194,7 @@ int bg_resident(int nt) {
 // resident-workgroup rounds).
 int bg_splits(int wgs, int nsb, int nt) {
     (void)bg_resident(nt);  // sets the kernel's LDS attribute
-    static int cus = 0;
-    if (!cus) {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-            n = 256;
-        cus = n;
-    }
+    const int cus = bg_cus();
     int best = 1;
     double best_t = 1e30;
     for (int sp = 1; sp <= std::min(16, std::max(1, nsb / 2)); sp++) {
@@ -896,25 +1215,50 @@ uint64_t bg_quant_bytes(int rows, int K) {
 
 }  // namespace
 
-// Grid of one launch: x workgroups of 8 tiles (SwiGLU: 4 channel tiles of
-// both matrices), y row blocks, z K splits.
-static void bg_grid(const int *n, int nseg, bool swiglu, int rows, int K, unsigned *gx, unsigned *gy, int *splits) {
-    unsigned x = 0;
-    if (swiglu)
-        x = (unsigned)((n[0] + 63) / 64);
-    else
-        for (int i = 0; i < nseg; i++) x += (unsigned)((n[i] + 16 * kBgWaves - 1) / (16 * kBgWaves));
-    *gx = x;
+// One launch: the channels (of each SwiGLU matrix) of a workgroup, its grid
+// (x channel blocks, y row blocks) and the K splits over grid z.
+struct BgPlan {
+    int few;  // bg_few_kernel: channel tiles to a wave; 0: bg_gemm_kernel
+    int channels;
+    unsigned gx, gy;
+    int splits;
+};
+static BgPlan bg_plan(const int *n, int nseg, bool swiglu, int rows, int K) {
+    BgPlan p{};
+    const int segs = swiglu ? 1 : nseg, nsb = K / 256;
+    auto blocks = [&](int channels) {
+        unsigned x = 0;
+        for (int i = 0; i < segs; i++) x += (unsigned)((n[i] + channels - 1) / channels);
+        return x;
+    };
+    int64_t all = 0;
+    for (int i = 0; i < nseg; i++) all += n[i];
+    if (bg_few_rows(rows, K, all)) {
+        // three channel tiles to a wave when with two the workgroups would be
+        // more than the CUs (40 rows of 2560 -> 2 x 9216: 28.6 us with three,
+        // 30.9 with two); else two, with K split until every CU has a
+        // workgroup (16 rows of 9216 -> 2560: 21.6 us in three splits, 23.1
+        // in two)
+        const int tile = swiglu ? 8 : 16, cus = bg_cus();
+        p.few = blocks(2 * tile) > (unsigned)cus ? 3 : 2;
+        p.channels = p.few * tile;
+        p.gx = blocks(p.channels);
+        p.gy = 1;
+        p.splits = p.few == 3 ? 1 : std::max(1, std::min(cus / (int)p.gx, nsb / 2));
+        return p;
+    }
+    // 8 tiles of 16 channels (SwiGLU: 4 of both matrices)
+    p.channels = (swiglu ? 64 : 16 * kBgWaves);
+    p.gx = blocks(p.channels);
     const int nt = bg_tiles(rows);
-    *gy = (unsigned)((rows + 16 * nt - 1) / (16 * nt));
-    *splits = bg_splits((int)(x * *gy), K / 256, nt);
+    p.gy = (unsigned)((rows + 16 * nt - 1) / (16 * nt));
+    p.splits = bg_splits((int)(p.gx * p.gy), nsb, nt);
+    return p;
 }
 
 void fused_gemm_rows_ws_parts(int rows, int K, const int *n, int nseg, bool swiglu, uint64_t *quant,
                               uint64_t *part) {
-    unsigned gx, gy;
-    int splits;
-    bg_grid(n, nseg, swiglu, rows, K, &gx, &gy, &splits);
+    const int splits = bg_plan(n, nseg, swiglu, rows, K).splits;
     int ncol = 0;
     for (int i = 0; i < nseg; i++) ncol += n[i];
     *quant = bg_quant_bytes(rows, K);
@@ -922,29 +1266,25 @@ void fused_gemm_rows_ws_parts(int rows, int K, const int *n, int nseg, bool swig
 }
 
 uint64_t fused_gemm_rows_ws(int rows, int K, const int *n, int nseg, bool swiglu) {
-    unsigned gx, gy;
-    int splits;
-    bg_grid(n, nseg, swiglu, rows, K, &gx, &gy, &splits);
-    int ncol = 0;
-    for (int i = 0; i < nseg; i++) ncol += n[i];
-    const uint64_t part = splits > 1 ? (uint64_t)splits * rows * ncol * 4 : 0;
-    return ((bg_quant_bytes(rows, K) + 255) & ~255ull) + part + 256;
+    uint64_t quant, part;
+    fused_gemm_rows_ws_parts(rows, K, n, nseg, swiglu, &quant, &part);
+    return ((quant + 255) & ~255ull) + part + 256;
 }
 
 // The arguments, grid and workspace view of one many-row launch.
-static void bg_setup(const FusedGemmArgs &a, void *ws, BgArgs &A, unsigned &gx, unsigned &gy,
-                     uint64_t part_off = 0) {
+static BgPlan bg_setup(const FusedGemmArgs &a, void *ws, BgArgs &A, uint64_t part_off = 0) {
     A = BgArgs{};
     A.f = a;
     A.q = bg_view(ws, a.rows, a.K);
     A.swiglu = a.epilogue == kEpiSwiglu ? 1 : 0;
-    // segment prefix in workgroups of 8 tiles (a workgroup never straddles two segments)
-    A.tiles[0] = 0;
-    for (int i = 0; i < a.nseg; i++) A.tiles[i + 1] = A.tiles[i] + (a.seg[i].n + 16 * kBgWaves - 1) / (16 * kBgWaves);
-    for (int i = a.nseg + 1; i <= kFusedMaxSeg; i++) A.tiles[i] = A.tiles[a.nseg];
     int nn[kFusedMaxSeg];
     for (int i = 0; i < a.nseg; i++) nn[i] = a.seg[i].n;
-    bg_grid(nn, a.nseg, A.swiglu != 0, a.rows, a.K, &gx, &gy, &A.splits);
+    const BgPlan p = bg_plan(nn, a.nseg, A.swiglu != 0, a.rows, a.K);
+    A.splits = p.splits;
+    // segment prefix in workgroups (a workgroup never straddles two segments)
+    A.tiles[0] = 0;
+    for (int i = 0; i < a.nseg; i++) A.tiles[i + 1] = A.tiles[i] + (a.seg[i].n + p.channels - 1) / p.channels;
+    for (int i = a.nseg + 1; i <= kFusedMaxSeg; i++) A.tiles[i] = A.tiles[a.nseg];
     A.cols[0] = 0;
     for (int i = 0; i < a.nseg; i++) A.cols[i + 1] = A.cols[i] + a.seg[i].n;
     for (int i = a.nseg + 1; i <= kFusedMaxSeg; i++) A.cols[i] = A.cols[a.nseg];
@@ -952,6 +1292,7 @@ static void bg_setup(const FusedGemmArgs &a, void *ws, BgArgs &A, unsigned &gx, 
     // common offset, past every member's quantized rows)
     A.part = reinterpret_cast<float *>(static_cast<uint8_t *>(ws) +
                                        (part_off ? part_off : (bg_quant_bytes(a.rows, a.K) + 255) & ~255ull));
+    return p;
 }
 
 static hipError_t bg_launch_prologue(const FusedGemmArgs &a, const BgQuant &q, const BgSrc &src, hipStream_t s) {
@@ -964,11 +1305,18 @@ static hipError_t bg_launch_prologue(const FusedGemmArgs &a, const BgQuant &q, c
 }
 
 // The GEMM, then (reduce and more than one split) the split reduction.
-static hipError_t bg_launch_gemm(const BgArgs &A, unsigned gx, unsigned gy, bool reduce, hipStream_t s) {
+static hipError_t bg_launch_gemm(const BgArgs &A, const BgPlan &p, bool reduce, hipStream_t s) {
     const FusedGemmArgs &a = A.f;
-    const dim3 grid(gx, gy, (unsigned)A.splits);
-    // (bg_grid's bg_resident call has set the kernel's LDS attribute)
-    if (bg_tiles(a.rows) == 5) bg_gemm_kernel<5><<<grid, kBgThreads, BgLds<5>::total, s>>>(A);
+    const dim3 grid(p.gx, p.gy, (unsigned)A.splits);
+    const int nr = bg_rows16(a.rows) / 16;
+    // (bg_plan's bg_resident call has set bg_gemm_kernel's LDS attribute)
+    if (p.few == 2 && nr == 1) bg_few_kernel<1, 2><<<grid, kFewThreads, 0, s>>>(A);
+    else if (p.few == 2 && nr == 2) bg_few_kernel<2, 2><<<grid, kFewThreads, 0, s>>>(A);
+    else if (p.few == 2) bg_few_kernel<3, 2><<<grid, kFewThreads, 0, s>>>(A);
+    else if (p.few == 3 && nr == 1) bg_few_kernel<1, 3><<<grid, kFewThreads, 0, s>>>(A);
+    else if (p.few == 3 && nr == 2) bg_few_kernel<2, 3><<<grid, kFewThreads, 0, s>>>(A);
+    else if (p.few == 3) bg_few_kernel<3, 3><<<grid, kFewThreads, 0, s>>>(A);
+    else if (bg_tiles(a.rows) == 5) bg_gemm_kernel<5><<<grid, kBgThreads, BgLds<5>::total, s>>>(A);
     else bg_gemm_kernel<3><<<grid, kBgThreads, BgLds<3>::total, s>>>(A);
     if (reduce && A.splits > 1) {
         const uint64_t nout = (uint64_t)a.rows * (A.swiglu ? a.seg[0].n : A.cols[a.nseg]);
@@ -979,10 +1327,9 @@ static hipError_t bg_launch_gemm(const BgArgs &A, unsigned gx, unsigned gy, bool
 
 hipError_t launch_fused_gemm_rows(const FusedGemmArgs &a, void *ws, hipStream_t s) {
     BgArgs A;
-    unsigned gx, gy;
-    bg_setup(a, ws, A, gx, gy);
+    const BgPlan p = bg_setup(a, ws, A);
     hipError_t err = bg_launch_prologue(a, A.q, BgSrc{}, s);
-    if (err == hipSuccess) err = bg_launch_gemm(A, gx, gy, true, s);
+    if (err == hipSuccess) err = bg_launch_gemm(A, p, true, s);
     return err;
 }
 
@@ -1003,13 +1350,12 @@ hipError_t launch_fused_gemm_rows_chain(const FusedGemmArgs *g, int n, void *ws,
     for (int i = 0; i < n; i++) {
         const FusedGemmArgs &a = g[i];
         BgArgs A;
-        unsigned gx, gy;
-        bg_setup(a, ws, A, gx, gy, part_off);
+        const BgPlan p = bg_setup(a, ws, A, part_off);
         const bool link = A.splits > 1 && i + 1 < n && bg_link(a, g[i + 1]);
         const bool defer = A.splits > 1 && i + 1 == n && defer_last && a.epilogue == kEpiResidual && a.nseg == 1 &&
                            a.seg[0].res != nullptr;
         hipError_t err = bg_launch_prologue(a, A.q, src, s);
-        if (err == hipSuccess) err = bg_launch_gemm(A, gx, gy, !(link || defer), s);
+        if (err == hipSuccess) err = bg_launch_gemm(A, p, !(link || defer), s);
         if (err != hipSuccess) return err;
         src = BgSrc{};
         if (link) {

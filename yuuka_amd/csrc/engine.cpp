@@ -243,7 +243,7 @@ struct Builder {
         int per = yk::fused_gemm_stream_rows((int)K0, norm != nullptr, gate != nullptr);
         if (per < 1) per = kRowBlock;
         // more than 8 rows: one launch of the many-row kernel (every weight
-        // read once per 64 rows)
+        // read once per block of 48 or 80 rows)
         if (rows > 8) per = (int)rows;
         const uint64_t blocks = (rows + per - 1) / per;
         for (uint64_t bi = 0; bi < blocks && st == YUUKA_OK; bi++) {

@@ -263,3 +263,28 @@ def test_truncated_batch_equals_requests_alone(dev, stream, B):
                                     request_base=b)
             alone, _ = _run(dev, stream, logits[b], drafts[b], one)
             assert res[b].tolist() == alone[0].tolist(), b
+
+
+# A tie group at the top-p cut, of fewer members than the counting order takes:
+# n equal logits below `head` larger ones, everything else out of reach. The
+# sampler adds the members' shares one by one, and six additions of 1/12 stay
+# below 0.5. One row cut in LDS whole, one through the binned candidates.
+@pytest.mark.parametrize("n,head,top_k,top_p", [
+    (12, 0, 0, 0.5), (14, 0, 0, 0.5), (24, 0, 0, 0.25), (24, 0, 0, 0.75), (12, 0, 12, 0.5), (30, 0, 12, 0.5),
+    (14, 0, 20, 0.5), (23, 3, 0, 0.75), (23, 3, 0, 0.5), (23, 3, 26, 0.75), (500, 0, 0, 0.3), (2, 1, 0, 0.9)])
+def test_top_p_cut_inside_a_small_tie_group(dev, stream, n, head, top_k, top_p):
+    rng = np.random.default_rng(n + head)
+    k = 2
+    totals = []
+    for V in (8192, 8193, 30000):
+        logits = np.full((k + 1, V), -100.0, np.float32)
+        ids = np.sort(rng.choice(8192, n + head, replace=False))
+        rng.shuffle(ids)
+        logits[:, ids[head:]] = 0.0
+        logits[:, ids[:head]] = 1.0 + np.arange(head)
+        drafts = np.array([np.sort(ids[head:])[n // 2 - 1], ids[0]], np.int32)
+        for step in range(2):
+            assert _check_truncated(dev, stream, logits, drafts, 1.0, top_k, top_p, 23, step) == 0
+        p = hip.accept_params(hip.ACCEPT_STOCHASTIC, 1, k, V, temperature=1.0, top_k=top_k, top_p=top_p, seed=23)
+        totals.append(_run(dev, stream, logits, drafts, p)[1][0, 0, 2])
+    assert max(totals) - min(totals) <= 1e-12 * totals[0]

@@ -859,6 +859,18 @@ __device__ int select_id(const float *p, int V, SelShared &s, uint32_t key, Cut 
     return id;
 }
 
+// Members of a boundary tie group (weight w each) that top_p keeps: they join
+// one by one, as the sampler's running sum adds their shares
+// (sampling.go:107-113), from the weight `before` ahead of the group.
+__device__ __forceinline__ uint32_t tie_members(double before, double w, double total, double top_p, uint32_t ties) {
+    double cum = before / total;
+    for (uint32_t i = 1; i < ties; i++) {
+        cum += w / total;
+        if (cum >= top_p) return i;
+    }
+    return ties;
+}
+
 // The cut of one row by radix selection over src. With `tail` (candidates of
 // one bin): the weight `before` lies ahead of src's elements, of `total`.
 __device__ __forceinline__ Cut radix_cut(const SelSrc src, SelShared &s, float mx, const Temp t, int top_k, float top_p,
@@ -938,22 +950,10 @@ __device__ __forceinline__ Cut radix_cut(const SelSrc src, SelShared &s, float m
             found = s.bucket >= 0;
         }
         if (found) {
-            // The tie group at the boundary: add its members one by one as the
-            // sampler's running sum does.
             if (threadIdx.x == 0) {
-                const uint32_t key = s.prefix;
                 const uint32_t ties = s.tc[s.bucket];
-                const double tot = s.total_w;
-                const double wt = soft_weight(key_value(key), mx, t);
-                double cum = s.before_w / tot;
-                uint32_t m = ties;
-                for (uint32_t i = 1; i <= ties; i++) {
-                    cum += wt / tot;
-                    if (cum >= (double)top_p) {
-                        m = i;
-                        break;
-                    }
-                }
+                const uint32_t m = tie_members(s.before_w, soft_weight(key_value(s.prefix), mx, t), s.total_w,
+                                               (double)top_p, ties);
                 s.before_c = m;  // kept members of the tie group
                 s.total_c = ties;
             }
@@ -1084,23 +1084,35 @@ __global__ __launch_bounds__(64 * kSelWaves) void accept_cut_kernel(const float 
             before = 0.0;
         }
         __syncthreads();
-        // the last kept member: the first one whose running share reaches
-        // top_p, else the lowest kept one
+        // the boundary is the first key whose members' weights reach top_p (none:
+        // the lowest kept member); of its members those up to the first one
+        // whose running share reaches it are kept, as in radix_cut
         const bool nucleus = top_p > 0.0f && top_p < 1.0f && total > 0.0 && !isinf(total);
-        bool reach = false;
-        if (nucleus) {
-            double ahead = 0.0;
-            for (int q = 0; q < n; q++) ahead += ord[q] > me ? wt[q] : 0.0;
-            reach = keep && before + ahead + w >= (double)top_p * total;
-        }
-        // (a first reach is the largest composite among those that reach)
-        __shared__ unsigned long long first_s;
+        const uint32_t key = (uint32_t)(me >> 32);
+        double ahead = 0.0, group = 0.0;
+        uint32_t place = 0u, ties = 0u;
+        if (nucleus && have)
+            for (int q = 0; q < n; q++) {
+                const unsigned long long o = ord[q];
+                const bool tie = (uint32_t)(o >> 32) == key;
+                ahead += !tie && o > me ? wt[q] : 0.0;
+                group += tie ? wt[q] : 0.0;
+                place += tie && o > me;
+                ties += tie;
+            }
+        const bool reach = nucleus && keep && before + ahead + group >= (double)top_p * total;
+        __shared__ unsigned long long first_s;  // the boundary key's first member
+        __shared__ uint32_t members_s;          // its kept members
         if (threadIdx.x == 0) first_s = 0ull;
         __syncthreads();
         if (reach) atomicMax(&first_s, me);
-        if (keep) atomicMin(&cut_s, me);
         __syncthreads();
-        const unsigned long long last = first_s ? first_s : cut_s;
+        const unsigned long long first = first_s;
+        if (have && me == first) members_s = tie_members(before + ahead, w, total, (double)top_p, ties);
+        __syncthreads();
+        if (keep && (!first || (key == (uint32_t)(first >> 32) && place < members_s))) atomicMin(&cut_s, me);
+        __syncthreads();
+        const unsigned long long last = cut_s;
         cut = Cut{(uint32_t)(last >> 32), (int32_t)~(uint32_t)last};
     } else {
         const SelSrc src{p, g.V, fits || direct ? list : nullptr, fits ? n : g.V, fits && top_k > 0};

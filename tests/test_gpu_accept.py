@@ -288,3 +288,14 @@ def test_top_p_cut_inside_a_small_tie_group(dev, stream, n, head, top_k, top_p):
         p = hip.accept_params(hip.ACCEPT_STOCHASTIC, 1, k, V, temperature=1.0, top_k=top_k, top_p=top_p, seed=23)
         totals.append(_run(dev, stream, logits, drafts, p)[1][0, 0, 2])
     assert max(totals) - min(totals) <= 1e-12 * totals[0]
+
+
+@pytest.mark.parametrize("V", [300, 9000])
+def test_difference_past_the_float_range_has_no_weight(dev, stream, V):
+    """logit - max overflows to -inf in float32; its weight is zero at every
+    finite temperature, also where the largest float over T is not far below 0."""
+    logits = np.full((2, V), -3e38, np.float32)
+    logits[:, 7] = 3e38
+    logits[:, 9] = 2.9e38
+    for top_k, top_p in [(0, 1.0), (0, 0.9), (5, 1.0), (5, 0.9)]:
+        assert _check_truncated(dev, stream, logits, np.array([9], np.int32), 1e38, top_k, top_p, 3, 1) == 0

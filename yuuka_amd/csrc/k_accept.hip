@@ -193,19 +193,19 @@ __device__ __forceinline__ bool in_cut(uint32_t key, int j, const Cut &c) {
     return key > c.key || (key == c.key && j <= c.id);
 }
 
-// The temperature as the weights use it: 1 / t rounded, and t for the
-// residual that makes the quotient below correctly rounded (up to its last
-// few denormals).
+// The temperature as the weights use it: 1 / t rounded, t for the residual
+// that makes the quotient below correctly rounded (up to its last few
+// denormals), and the quotient of -inf (a difference past the float range).
 struct Temp {
-    double t, rt;
+    double t, rt, low;
 };
 
-// (logit - max) / T; -inf stays out of the residual.
+// float64(logit - max) / T.
 __device__ __forceinline__ double exponent_of(float l, float mx, const Temp &t) {
-    float d = l - mx;
-    d = d == -INFINITY ? -3.4e38f : d;
+    const float d = l - mx;
     const double a = (double)d, q = a * t.rt;
-    return fma(fma(-q, t.t, a), t.rt, q);
+    const double x = fma(fma(-q, t.t, a), t.rt, q);
+    return d == -INFINITY ? t.low : x;
 }
 
 // exp(x) for x <= 0 (NaN stays NaN): 2^k e^r with r = x - k ln 2 in two FMA
@@ -1633,7 +1633,7 @@ hipError_t launch_verify_accept(const float *logits, const int32_t *drafts, int3
     double *wdraft = sums + n;
     const bool stochastic = p.mode == YUUKA_ACCEPT_STOCHASTIC && p.temperature > 0.0f && p.top_k != 1;
     const double td = stochastic ? std::min((double)p.temperature, 1e300) : 1.0;
-    const Temp t{td, 1.0 / td};
+    const Temp t{td, 1.0 / td, -INFINITY / (stochastic ? (double)p.temperature : 1.0)};
     // top_p 0 means off (sampling.go:46-48); top_k at or above the vocabulary keeps everything.
     const bool top_k_on = p.top_k > 1 && p.top_k < p.vocab;
     const bool top_p_on = p.top_p > 0.0f && p.top_p < 1.0f;

@@ -35,6 +35,7 @@
 #include <climits>
 #include <type_traits>
 
+#include "accept_math.h"
 #include "internal.h"
 
 namespace yk {
@@ -193,82 +194,16 @@ __device__ __forceinline__ bool in_cut(uint32_t key, int j, const Cut &c) {
     return key > c.key || (key == c.key && j <= c.id);
 }
 
-// The temperature as the weights use it: 1 / t rounded, t for the residual
-// that makes the quotient below correctly rounded (up to its last few
-// denormals), and the quotient of -inf (a difference past the float range).
-struct Temp {
-    double t, rt, low;
-};
-
-// float64(logit - max) / T.
-__device__ __forceinline__ double exponent_of(float l, float mx, const Temp &t) {
-    const float d = l - mx;
-    const double a = (double)d, q = a * t.rt;
-    const double x = fma(fma(-q, t.t, a), t.rt, q);
-    return d == -INFINITY ? t.low : x;
+// The exponential's table in LDS, by the first threads of a workgroup
+// (complete at its next barrier).
+__device__ __forceinline__ void load_exp_tab(ExpEntry *tab) {
+    if (threadIdx.x < 16) tab[threadIdx.x] = kExpTab[threadIdx.x];
 }
 
-// exp(x) for x <= 0 (NaN stays NaN): 2^k e^r with r = x - k ln 2 in two FMA
-// steps (|r| <= 0.35) and the Taylor series of e^r to r^13 (its remainder is
-// below 5e-18).
-__device__ __forceinline__ double exp_nonpos(double x) {
-    const double k = rint(x * 0x1.71547652b82fep+0);
-    const double r = fma(k, -0x1.abc9e3b39803fp-56, fma(k, -0x1.62e42fefa39efp-1, x));
-    double p = 1.0 / 6227020800.0;
-    p = fma(p, r, 1.0 / 479001600.0);
-    p = fma(p, r, 1.0 / 39916800.0);
-    p = fma(p, r, 1.0 / 3628800.0);
-    p = fma(p, r, 1.0 / 362880.0);
-    p = fma(p, r, 1.0 / 40320.0);
-    p = fma(p, r, 1.0 / 5040.0);
-    p = fma(p, r, 1.0 / 720.0);
-    p = fma(p, r, 1.0 / 120.0);
-    p = fma(p, r, 1.0 / 24.0);
-    p = fma(p, r, 1.0 / 6.0);
-    p = fma(p, r, 0.5);
-    p = fma(p, r, 1.0);
-    p = fma(p, r, 1.0);
-    const double e = ldexp(p, (int)k);
-    return x < -760.0 ? 0.0 : e;  // below the smallest denormal (k may be anything there)
-}
-
-// exp(x) for x <= 0 for the pass that weighs a whole vocabulary, which its
-// float64 operations bound: 2^(k/16) (and its rounding error) from a table
-// in LDS, e^r for |r| <= ln 2 / 32 to r^7 (remainder below 2e-18). Within
-// 0.6 ulp; with the plain series the pass took 51 us at 144 rows of 151936.
-__constant__ double2 kExpTab[16] = {
-    {0x1.0000000000000p+0, 0x0.0p+0}, {0x1.0b5586cf9890fp+0, 0x1.8a62e4adc610bp-54},
-    {0x1.172b83c7d517bp+0, -0x1.19041b9d78a76p-55}, {0x1.2387a6e756238p+0, 0x1.9b07eb6c70573p-54},
-    {0x1.306fe0a31b715p+0, 0x1.6f46ad23182e4p-55}, {0x1.3dea64c123422p+0, 0x1.ada0911f09ebcp-55},
-    {0x1.4bfdad5362a27p+0, 0x1.d4397afec42e2p-56}, {0x1.5ab07dd485429p+0, 0x1.6324c054647adp-54},
-    {0x1.6a09e667f3bcdp+0, -0x1.bdd3413b26456p-54}, {0x1.7a11473eb0187p+0, -0x1.41577ee04992fp-55},
-    {0x1.8ace5422aa0dbp+0, 0x1.6e9f156864b27p-54}, {0x1.9c49182a3f090p+0, 0x1.c7c46b071f2bep-56},
-    {0x1.ae89f995ad3adp+0, 0x1.7a1cd345dcc81p-54}, {0x1.c199bdd85529cp+0, 0x1.11065895048ddp-55},
-    {0x1.d5818dcfba487p+0, 0x1.2ed02d75b3707p-55}, {0x1.ea4afa2a490dap+0, -0x1.e9c23179c2893p-54}};
-__device__ __forceinline__ double exp_nonpos_tab(double x, const double2 *tab) {
-    const double k = rint(x * 0x1.71547652b82fep+4);
-    const double r = fma(k, -0x1.abc9e3b39803fp-60, fma(k, -0x1.62e42fefa39efp-5, x));
-    double p = fma(r, 1.0 / 5040.0, 1.0 / 720.0);
-    p = fma(p, r, 1.0 / 120.0);
-    p = fma(p, r, 1.0 / 24.0);
-    p = fma(p, r, 1.0 / 6.0);
-    p = fma(p, r, 0.5);
-    p = fma(p, r, 1.0);
-    const int ki = (int)k;
-    const double2 f = tab[ki & 15];
-    const double e = ldexp(f.x + fma(f.x, p * r, f.y), ki >> 4);
-    return x < -760.0 ? 0.0 : e;
-}
-
-// exp(float64(logit - max) / T) (sampling.go:97) of a valid logit.
-__device__ __forceinline__ double soft_weight(float l, float mx, const Temp &t) {
-    return exp_nonpos(exponent_of(l, mx, t));
-}
-
-// The same, zero outside the cut.
-__device__ __forceinline__ double weight_of(float l, int j, float mx, const Temp &t, const Cut &c) {
+// The weight of a logit, zero outside the cut.
+__device__ __forceinline__ double weight_of(float l, int j, float mx, const Temp &t, const Cut &c, const ExpEntry *tab) {
     if (!valid_logit(l) || !in_cut(order_key(l), j, c)) return 0.0;
-    return soft_weight(l, mx, t);
+    return soft_weight(l, mx, t, tab);
 }
 
 // Wave 0 of a workgroup: the row's maximum and its first index over the
@@ -294,8 +229,8 @@ __global__ __launch_bounds__(256) void accept_weights_kernel(const float *__rest
     const int c = blockIdx.x, row = blockIdx.y, b = blockIdx.z;
     const float *p = row_ptr(logits, g, b, row);
     __shared__ float mx_s;
-    __shared__ double2 tab[16];
-    if (threadIdx.x < 16) tab[threadIdx.x] = kExpTab[threadIdx.x];
+    __shared__ ExpEntry tab[16];
+    load_exp_tab(tab);
     if (threadIdx.x < 64) {
         const Stat s = wave_best(stats + ((uint64_t)b * g.R + row) * g.C, g.C);
         if (threadIdx.x == 0) mx_s = s.v;
@@ -307,7 +242,7 @@ __global__ __launch_bounds__(256) void accept_weights_kernel(const float *__rest
     const int end = min(begin + g.L, g.V);
     double acc = 0.0;
     auto weigh = [&](float l) __attribute__((always_inline)) {
-        const double w = exp_nonpos_tab(exponent_of(l, mx, t), tab);
+        const double w = soft_weight(l, mx, t, tab);
         return valid_logit(l) ? w : 0.0;
     };
     // eight logit loads in flight per thread; the sum keeps index order
@@ -446,8 +381,8 @@ __global__ __launch_bounds__(64 * kBinWaves) void accept_bins_kernel(const float
     extern __shared__ __attribute__((aligned(16))) uint8_t bins_dyn[];
     T *hist = reinterpret_cast<T *>(bins_dyn);  // [wave][NB]
     __shared__ float mx_s, scale_s;
-    __shared__ double2 tab[16];
-    if (!COUNT && threadIdx.x < 16) tab[threadIdx.x] = kExpTab[threadIdx.x];
+    __shared__ ExpEntry tab[16];
+    if (!COUNT) load_exp_tab(tab);
     constexpr int kT = 64 * kBinWaves;
     const int c = blockIdx.x, row = blockIdx.y, b = blockIdx.z;
     const float *p = row_ptr(logits, g, b, row);
@@ -488,7 +423,7 @@ __global__ __launch_bounds__(64 * kBinWaves) void accept_bins_kernel(const float
             for (int u0 = 0; u0 < kU; u0 += kW) {
                 double w[kW];
 #pragma unroll
-                for (int u = 0; u < kW; u++) w[u] = exp_nonpos_tab(exponent_of(lv[u0 + u], mx, t), tab);
+                for (int u = 0; u < kW; u++) w[u] = soft_weight(lv[u0 + u], mx, t, tab);
 #pragma unroll
                 for (int u = 0; u < kW; u++) {
                     const float l = lv[u0 + u];
@@ -526,6 +461,8 @@ __global__ __launch_bounds__(256) void accept_collect_kernel(const float *__rest
     __shared__ int best_i_s, bnd_s;
     __shared__ T wave_tot[4];
     __shared__ T before_s;
+    __shared__ ExpEntry tab[16];
+    if (!COUNT) load_exp_tab(tab);
     const int c = blockIdx.x, row = blockIdx.y, b = blockIdx.z;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const float *p = row_ptr(logits, g, b, row);
@@ -576,7 +513,7 @@ __global__ __launch_bounds__(256) void accept_collect_kernel(const float *__rest
     double wd = 0.0;
     int dbin = tg.NB;
     if (!COUNT && d >= 0 && d < g.V && valid_logit(p[d])) {
-        wd = soft_weight(p[d], mx, t);
+        wd = soft_weight(p[d], mx, t, tab);
         dbin = bin_of(p[d], mx, scale, tg.NB);
     }
     const double total = (double)tot + wd;
@@ -665,6 +602,7 @@ struct SelShared {
     double total_w;     // all weight of the first pass
     uint32_t total_c;
     int id;             // result of an id selection
+    ExpEntry tab[16];
 };
 
 // The elements a selection runs over: a candidate list in LDS, or (list
@@ -713,7 +651,7 @@ __device__ __forceinline__ void hist_pass(const SelSrc &src, float mx, const Tem
         if (!sel(k, j)) return;
         const int b = (k >> shift) & 255u;
         atomicAdd(&s.cnt[wave][b], 1u);
-        if (W) unsafeAtomicAdd(&s.wsum[wave][b], soft_weight(l, mx, t));
+        if (W) unsafeAtomicAdd(&s.wsum[wave][b], soft_weight(l, mx, t, s.tab));
     });
     __syncthreads();
     if (threadIdx.x < 256) {
@@ -952,7 +890,7 @@ __device__ __forceinline__ Cut radix_cut(const SelSrc src, SelShared &s, float m
         if (found) {
             if (threadIdx.x == 0) {
                 const uint32_t ties = s.tc[s.bucket];
-                const uint32_t m = tie_members(s.before_w, soft_weight(key_value(s.prefix), mx, t), s.total_w,
+                const uint32_t m = tie_members(s.before_w, soft_weight(key_value(s.prefix), mx, t, s.tab), s.total_w,
                                                (double)top_p, ties);
                 s.before_c = m;  // kept members of the tie group
                 s.total_c = ties;
@@ -1000,6 +938,7 @@ __global__ __launch_bounds__(64 * kSelWaves) void accept_cut_kernel(const float 
     extern __shared__ __attribute__((aligned(16))) uint8_t cut_dyn[];
     Member *list = reinterpret_cast<Member *>(cut_dyn);
     RowCut in = rc;
+    load_exp_tab(s.tab);
     if (direct) {
         __shared__ Stat best_s;
         for (int j = threadIdx.x; j < g.V; j += 64 * kSelWaves) list[j] = Member{p[j], j};
@@ -1076,7 +1015,7 @@ __global__ __launch_bounds__(64 * kSelWaves) void accept_cut_kernel(const float 
             for (int q = 0; q < n; q++) ahead += ord[q] > me;
             keep = have && ahead < (uint32_t)top_k;
         }
-        if (keep) w = soft_weight(list[i].l, mx, t);
+        if (keep) w = soft_weight(list[i].l, mx, t, s.tab);
         if (have) wt[i] = keep ? w : 0.0;
         double total = in.total, before = in.before;
         if (top_k > 0) {
@@ -1123,7 +1062,7 @@ __global__ __launch_bounds__(64 * kSelWaves) void accept_cut_kernel(const float 
     const SelSrc src{p, g.V, fits || direct ? list : nullptr, fits ? n : g.V, false};
     double sum = 0.0;
     for_each(src, [&](float l, int j) __attribute__((always_inline)) {
-        if (j != d && in_cut(order_key(l), j, cut)) sum += soft_weight(l, mx, t);
+        if (j != d && in_cut(order_key(l), j, cut)) sum += soft_weight(l, mx, t, s.tab);
     });
     sum = block_sum(sum, waves);
     if (threadIdx.x == 0) {
@@ -1131,7 +1070,7 @@ __global__ __launch_bounds__(64 * kSelWaves) void accept_cut_kernel(const float 
         rc.best_i = in.best_i;
         rc.cut = cut;
         rc.rest = sum + (fits && top_k <= 0 ? in.before_rest : 0.0);
-        rc.wd = d >= 0 && d < g.V ? weight_of(p[d], d, mx, t, cut) : 0.0;
+        rc.wd = d >= 0 && d < g.V ? weight_of(p[d], d, mx, t, cut, s.tab) : 0.0;
     }
 }
 
@@ -1184,7 +1123,7 @@ __global__ __launch_bounds__(256) void router_normal_kernel(float *__restrict__ 
 // target lies beyond the chunk's own sum (rounding), with *last the last
 // positive-weight index of the chunk.
 __device__ int scan_chunk(const float *p, int begin, int end, int d, float mx, const Temp &t, const Cut &cut,
-                          double target, double *shared_prefix, int *shared_pick) {
+                          const ExpEntry *tab, double target, double *shared_prefix, int *shared_pick) {
     const int len = end - begin;
     const int per = (len + 255) / 256;
     const int lo = begin + threadIdx.x * per;
@@ -1197,10 +1136,10 @@ __device__ int scan_chunk(const float *p, int begin, int end, int d, float mx, c
         for (int u = 0; u < 8; u++) l[u] = p[j + u];
 #pragma unroll
         for (int u = 0; u < 8; u++)
-            if (j + u != d) local += weight_of(l[u], j + u, mx, t, cut);
+            if (j + u != d) local += weight_of(l[u], j + u, mx, t, cut, tab);
     }
     for (; j < hi; j++)
-        if (j != d) local += weight_of(p[j], j, mx, t, cut);
+        if (j != d) local += weight_of(p[j], j, mx, t, cut, tab);
     shared_prefix[threadIdx.x] = local;
     if (threadIdx.x == 0) *shared_pick = -1;
     __syncthreads();
@@ -1222,7 +1161,7 @@ __device__ int scan_chunk(const float *p, int begin, int end, int d, float mx, c
     if (run <= target && target < run + local) {
         for (int j = lo; j < hi; j++) {
             if (j == d) continue;
-            const double w = weight_of(p[j], j, mx, t, cut);
+            const double w = weight_of(p[j], j, mx, t, cut, tab);
             if (w <= 0.0) continue;
             run += w;
             if (target < run) {
@@ -1232,7 +1171,7 @@ __device__ int scan_chunk(const float *p, int begin, int end, int d, float mx, c
         }
         if (*shared_pick < 0) {  // rounding at the boundary: last positive weight
             for (int j = hi - 1; j >= lo; j--)
-                if (j != d && weight_of(p[j], j, mx, t, cut) > 0.0) {
+                if (j != d && weight_of(p[j], j, mx, t, cut, tab) > 0.0) {
                     *shared_pick = j;
                     break;
                 }
@@ -1252,6 +1191,7 @@ __global__ __launch_bounds__(256) void accept_finalize_kernel(
     if (step_dev) step = *step_dev;
     const uint32_t request = request_base + (uint32_t)b;
     __shared__ double prefix[256];
+    __shared__ ExpEntry tab[16];
     __shared__ int pick;
     __shared__ int decided_next;
     __shared__ int accepted_s;
@@ -1260,6 +1200,7 @@ __global__ __launch_bounds__(256) void accept_finalize_kernel(
     __shared__ double row_rest_s[256];
     __shared__ float row_p0_s[256];  // logit 0 of each row
     __shared__ int row_d_s[256];     // each row's draft (-1 on the bonus row)
+    load_exp_tab(tab);
     if (threadIdx.x == 0) {
         decided_next = -1;
         accepted_s = 0;
@@ -1387,7 +1328,7 @@ __global__ __launch_bounds__(256) void accept_finalize_kernel(
         if (action == 2) {
             const int d = row < g.k ? drafts[(uint64_t)b * g.ds + row] : -1;
             const int begin = cstar * g.L;
-            const int j = scan_chunk(p, begin, min(begin + g.L, g.V), d, mx_s, t, Cut{0u, INT_MAX}, target_s, prefix, &pick);
+            const int j = scan_chunk(p, begin, min(begin + g.L, g.V), d, mx_s, t, Cut{0u, INT_MAX}, tab, target_s, prefix, &pick);
             if (threadIdx.x == 0) decided_next = j >= 0 ? j : best_s.i;
         }
         break;
@@ -1481,6 +1422,8 @@ __global__ __launch_bounds__(256) void accept_resample_kernel(const float *__res
     const int c = blockIdx.x, b = blockIdx.y;
     __shared__ int row_s, d_s;
     __shared__ double ws[4];
+    __shared__ ExpEntry tab[16];
+    load_exp_tab(tab);
     if (step_dev) step = *step_dev;
     if (threadIdx.x < 64) {
         const Decision dec = decide(logits, g, b, drafts, area, seed, step, request_base + (uint32_t)b, forced, nullptr);
@@ -1505,7 +1448,7 @@ __global__ __launch_bounds__(256) void accept_resample_kernel(const float *__res
         for (int u = 0; u < kU; u++) l[u] = j0 + u * 256 < end ? p[j0 + u * 256] : NAN;
 #pragma unroll
         for (int u = 0; u < kU; u++)
-            if (j0 + u * 256 != d) acc += weight_of(l[u], j0 + u * 256, mx, t, cut);
+            if (j0 + u * 256 != d) acc += weight_of(l[u], j0 + u * 256, mx, t, cut, tab);
     }
     for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
     if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = acc;
@@ -1527,6 +1470,8 @@ __global__ __launch_bounds__(256) void accept_pick_kernel(const float *__restric
     __shared__ int pick, cstar_s;
     __shared__ double target_s;
     __shared__ Decision dec_s;
+    __shared__ ExpEntry tab[16];
+    load_exp_tab(tab);
     if (step_dev) step = *step_dev;
     if (threadIdx.x < 64) {
         // RC <= 64: lane c's chunk; the target's chunk is the last one whose
@@ -1555,7 +1500,7 @@ __global__ __launch_bounds__(256) void accept_pick_kernel(const float *__restric
         const RowCut &rc = row_cut(area, g, b, dec.row);
         const int c = cstar_s;
         const int j = scan_chunk(row_ptr(logits, g, b, dec.row), (int)((int64_t)g.V * c / RC),
-                                 (int)((int64_t)g.V * (c + 1) / RC), dec.d, rc.best_v, t, rc.cut, target_s, prefix, &pick);
+                                 (int)((int64_t)g.V * (c + 1) / RC), dec.d, rc.best_v, t, rc.cut, tab, target_s, prefix, &pick);
         next = j >= 0 ? j : rc.best_i;
     }
     if (threadIdx.x == 0) {
@@ -1632,8 +1577,7 @@ hipError_t launch_verify_accept(const float *logits, const int32_t *drafts, int3
     double *sums = reinterpret_cast<double *>(base + ((n * sizeof(Stat) + 255) & ~255ull));
     double *wdraft = sums + n;
     const bool stochastic = p.mode == YUUKA_ACCEPT_STOCHASTIC && p.temperature > 0.0f && p.top_k != 1;
-    const double td = stochastic ? std::min((double)p.temperature, 1e300) : 1.0;
-    const Temp t{td, 1.0 / td, -INFINITY / (stochastic ? (double)p.temperature : 1.0)};
+    const Temp t = make_temp(stochastic ? p.temperature : 1.0f);
     // top_p 0 means off (sampling.go:46-48); top_k at or above the vocabulary keeps everything.
     const bool top_k_on = p.top_k > 1 && p.top_k < p.vocab;
     const bool top_p_on = p.top_p > 0.0f && p.top_p < 1.0f;

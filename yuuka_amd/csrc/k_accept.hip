@@ -194,10 +194,11 @@ __device__ __forceinline__ bool in_cut(uint32_t key, int j, const Cut &c) {
     return key > c.key || (key == c.key && j <= c.id);
 }
 
-// The exponential's table in LDS, by the first threads of a workgroup
-// (complete at its next barrier).
-__device__ __forceinline__ void load_exp_tab(ExpEntry *tab) {
-    if (threadIdx.x < 16) tab[threadIdx.x] = kExpTab[threadIdx.x];
+// The exponential's table in LDS: a thread's entry is loaded at a kernel's
+// start and put down just before its first barrier, behind its other loads.
+__device__ __forceinline__ ExpEntry exp_entry() { return kExpTab[threadIdx.x & 15]; }
+__device__ __forceinline__ void put_exp_entry(ExpEntry *tab, const ExpEntry &e) {
+    if (threadIdx.x < 16) tab[threadIdx.x] = e;
 }
 
 // The weight of a logit, zero outside the cut.
@@ -230,11 +231,12 @@ __global__ __launch_bounds__(256) void accept_weights_kernel(const float *__rest
     const float *p = row_ptr(logits, g, b, row);
     __shared__ float mx_s;
     __shared__ ExpEntry tab[16];
-    load_exp_tab(tab);
+    const ExpEntry entry = exp_entry();
     if (threadIdx.x < 64) {
         const Stat s = wave_best(stats + ((uint64_t)b * g.R + row) * g.C, g.C);
         if (threadIdx.x == 0) mx_s = s.v;
     }
+    put_exp_entry(tab, entry);
     __syncthreads();
     const float mx = mx_s;
     const int d = row < g.k ? drafts[(uint64_t)b * g.ds + row] : -1;
@@ -382,7 +384,7 @@ __global__ __launch_bounds__(64 * kBinWaves) void accept_bins_kernel(const float
     T *hist = reinterpret_cast<T *>(bins_dyn);  // [wave][NB]
     __shared__ float mx_s, scale_s;
     __shared__ ExpEntry tab[16];
-    if (!COUNT) load_exp_tab(tab);
+    const ExpEntry entry = exp_entry();
     constexpr int kT = 64 * kBinWaves;
     const int c = blockIdx.x, row = blockIdx.y, b = blockIdx.z;
     const float *p = row_ptr(logits, g, b, row);
@@ -402,6 +404,7 @@ __global__ __launch_bounds__(64 * kBinWaves) void accept_bins_kernel(const float
             scale_s = sc;
         }
     }
+    put_exp_entry(tab, entry);
     __syncthreads();
     const float mx = mx_s, scale = scale_s;
     const int d = !COUNT && row < g.k ? drafts[(uint64_t)b * g.ds + row] : -1;
@@ -462,7 +465,7 @@ __global__ __launch_bounds__(256) void accept_collect_kernel(const float *__rest
     __shared__ T wave_tot[4];
     __shared__ T before_s;
     __shared__ ExpEntry tab[16];
-    if (!COUNT) load_exp_tab(tab);
+    const ExpEntry entry = exp_entry();
     const int c = blockIdx.x, row = blockIdx.y, b = blockIdx.z;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const float *p = row_ptr(logits, g, b, row);
@@ -501,6 +504,7 @@ __global__ __launch_bounds__(256) void accept_collect_kernel(const float *__rest
     T exc = __shfl_up(inc, 1);
     if (lane == 0) exc = (T)0;
     if (lane == 63) wave_tot[wave] = inc;
+    put_exp_entry(tab, entry);
     __syncthreads();
     const float mx = mx_s, scale = scale_s;
     T tot = (T)0;
@@ -919,7 +923,7 @@ __device__ __forceinline__ double block_sum(double v, double *waves) {
 
 // One workgroup per row: the exact cut, and the kept weight without the
 // draft and of the draft. Up to kRankMost candidates are put in order by
-// counting (thread i adds up what lies ahead of candidate i); more take the
+// counting (thread i counts what lies ahead of candidate i); more take the
 // radix selection. `direct`: no candidates were collected, the row itself is
 // taken (into LDS).
 __global__ __launch_bounds__(64 * kSelWaves) void accept_cut_kernel(const float *__restrict__ logits, Geo g, TruncGeo tg,
@@ -933,12 +937,11 @@ __global__ __launch_bounds__(64 * kSelWaves) void accept_cut_kernel(const float 
     __shared__ SelShared s;
     __shared__ double waves[kSelWaves];
     __shared__ uint32_t seg_at[260];
-    __shared__ unsigned long long cut_s;
-    __shared__ int n_s;
+    __shared__ int n_s, end_s, last_s;
     extern __shared__ __attribute__((aligned(16))) uint8_t cut_dyn[];
     Member *list = reinterpret_cast<Member *>(cut_dyn);
     RowCut in = rc;
-    load_exp_tab(s.tab);
+    const ExpEntry entry = exp_entry();
     if (direct) {
         __shared__ Stat best_s;
         for (int j = threadIdx.x; j < g.V; j += 64 * kSelWaves) list[j] = Member{p[j], j};
@@ -951,6 +954,7 @@ __global__ __launch_bounds__(64 * kSelWaves) void accept_cut_kernel(const float 
         in.best_v = best_s.v;
         in.best_i = best_s.i;
     }
+    put_exp_entry(s.tab, entry);
     const float mx = in.best_v;
     if (in.status == kCutAll) return;  // the defaults of collect hold
     const int d = row < g.k ? drafts[(uint64_t)b * g.ds + row] : -1;
@@ -999,59 +1003,62 @@ __global__ __launch_bounds__(64 * kSelWaves) void accept_cut_kernel(const float 
     Cut cut{0u, INT_MAX};
     if (fits && n <= kRankMost) {
         // composite order: a larger (key, ~id) is ahead
-        unsigned long long *ord = reinterpret_cast<unsigned long long *>(&s.wsum[0][0]);
-        double *wt = reinterpret_cast<double *>(&s.wsum[0][0]) + kRankMost;
-        const int i = threadIdx.x;
+        unsigned long long *ord = reinterpret_cast<unsigned long long *>(&s.wsum[0][0]), *sorted = ord + kRankMost;
+        double *wt = reinterpret_cast<double *>(sorted + kRankMost);
+        const int i = threadIdx.x, wave = i >> 6, lane = i & 63;
         const bool have = i < n;
-        const unsigned long long me =
-            have ? ((unsigned long long)order_key(list[i].l) << 32) | (uint32_t)~(uint32_t)list[i].j : 0ull;
-        double w = 0.0;
-        if (have) ord[i] = me;
-        if (threadIdx.x == 0) cut_s = ~0ull;
+        // with top-k the candidates are everything down to the boundary bin
+        const int kept = top_k > 0 ? min(n, top_k) : n;
+        if (have) ord[i] = ((unsigned long long)order_key(list[i].l) << 32) | (uint32_t)~(uint32_t)list[i].j;
+        if (i == 0) end_s = kept - 1;
         __syncthreads();
-        bool keep = have;
-        if (top_k > 0) {  // the candidates are everything down to the boundary bin
-            uint32_t ahead = 0u;
-            for (int q = 0; q < n; q++) ahead += ord[q] > me;
-            keep = have && ahead < (uint32_t)top_k;
-        }
-        if (keep) w = soft_weight(list[i].l, mx, t, s.tab);
-        if (have) wt[i] = keep ? w : 0.0;
-        double total = in.total, before = in.before;
-        if (top_k > 0) {
-            total = block_sum(w, waves);
-            before = 0.0;
+        if (have) {
+            const unsigned long long me = ord[i];
+            int at = 0;
+            for (int q = 0; q < n; q++) at += ord[q] > me;
+            sorted[at] = me;
+            wt[at] = at < kept ? soft_weight(list[i].l, mx, t, s.tab) : 0.0;
         }
         __syncthreads();
-        // the boundary is the first key whose members' weights reach top_p (none:
-        // the lowest kept member); of its members those up to the first one
-        // whose running share reaches it are kept, as in radix_cut
-        const bool nucleus = top_p > 0.0f && top_p < 1.0f && total > 0.0 && !isinf(total);
-        const uint32_t key = (uint32_t)(me >> 32);
-        double ahead = 0.0, group = 0.0;
-        uint32_t place = 0u, ties = 0u;
-        if (nucleus && have)
-            for (int q = 0; q < n; q++) {
-                const unsigned long long o = ord[q];
-                const bool tie = (uint32_t)(o >> 32) == key;
-                ahead += !tie && o > me ? wt[q] : 0.0;
-                group += tie ? wt[q] : 0.0;
-                place += tie && o > me;
-                ties += tie;
+        // thread i: the i-th member, the weights up to it and before it
+        const double w = have ? wt[i] : 0.0;
+        const uint32_t key = have ? (uint32_t)(sorted[i] >> 32) : 0u;
+        double inc = w;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const double v = __shfl_up(inc, off);
+            if (lane >= off) inc += v;
+        }
+        double exc = __shfl_up(inc, 1);
+        if (lane == 0) exc = 0.0;
+        // (members of one wave only: the others have nothing to decide)
+        double sum = __shfl(inc, 63), base = 0.0;
+        if (n > 64) {
+            if (lane == 63) waves[wave] = inc;
+            __syncthreads();
+            sum = 0.0;
+            for (int q = 0; q < kSelWaves; q++) {
+                if (q == wave) base = sum;
+                sum += waves[q];
             }
-        const bool reach = nucleus && keep && before + ahead + group >= (double)top_p * total;
-        __shared__ unsigned long long first_s;  // the boundary key's first member
-        __shared__ uint32_t members_s;          // its kept members
-        if (threadIdx.x == 0) first_s = 0ull;
+        }
+        const double before = top_k > 0 ? 0.0 : in.before, total = top_k > 0 ? sum : in.total;
+        inc += base;
+        exc += base;
+        // the boundary is the first key whose members' weights reach top_p (none:
+        // the last key); of its members those up to the first one whose running
+        // share reaches it are kept, as in radix_cut
+        const bool nucleus = top_p > 0.0f && top_p < 1.0f && total > 0.0 && !isinf(total);
+        if (nucleus && i < kept && (i + 1 == kept || (uint32_t)(sorted[i + 1] >> 32) != key) &&
+            before + inc >= (double)top_p * total)
+            atomicMin(&end_s, i);
         __syncthreads();
-        if (reach) atomicMax(&first_s, me);
+        const int end = end_s;
+        // the first member of the boundary key
+        if (i <= end && key == (uint32_t)(sorted[end] >> 32) && (i == 0 || (uint32_t)(sorted[i - 1] >> 32) != key))
+            last_s = !nucleus ? end : i - 1 + (int)tie_members(before + exc, w, total, (double)top_p, (uint32_t)(end - i + 1));
         __syncthreads();
-        const unsigned long long first = first_s;
-        if (have && me == first) members_s = tie_members(before + ahead, w, total, (double)top_p, ties);
-        __syncthreads();
-        if (keep && (!first || (key == (uint32_t)(first >> 32) && place < members_s))) atomicMin(&cut_s, me);
-        __syncthreads();
-        const unsigned long long last = cut_s;
+        const unsigned long long last = sorted[last_s];
         cut = Cut{(uint32_t)(last >> 32), (int32_t)~(uint32_t)last};
     } else {
         const SelSrc src{p, g.V, fits || direct ? list : nullptr, fits ? n : g.V, fits && top_k > 0};
@@ -1200,7 +1207,7 @@ __global__ __launch_bounds__(256) void accept_finalize_kernel(
     __shared__ double row_rest_s[256];
     __shared__ float row_p0_s[256];  // logit 0 of each row
     __shared__ int row_d_s[256];     // each row's draft (-1 on the bonus row)
-    load_exp_tab(tab);
+    const ExpEntry entry = exp_entry();
     if (threadIdx.x == 0) {
         decided_next = -1;
         accepted_s = 0;
@@ -1230,6 +1237,7 @@ __global__ __launch_bounds__(256) void accept_finalize_kernel(
             }
         }
     }
+    put_exp_entry(tab, entry);
     __syncthreads();
     for (int row = 0; row <= g.k; row++) {
         const float *p = row_ptr(logits, g, b, row);
@@ -1423,7 +1431,7 @@ __global__ __launch_bounds__(256) void accept_resample_kernel(const float *__res
     __shared__ int row_s, d_s;
     __shared__ double ws[4];
     __shared__ ExpEntry tab[16];
-    load_exp_tab(tab);
+    const ExpEntry entry = exp_entry();
     if (step_dev) step = *step_dev;
     if (threadIdx.x < 64) {
         const Decision dec = decide(logits, g, b, drafts, area, seed, step, request_base + (uint32_t)b, forced, nullptr);
@@ -1432,6 +1440,7 @@ __global__ __launch_bounds__(256) void accept_resample_kernel(const float *__res
             d_s = dec.d;
         }
     }
+    put_exp_entry(tab, entry);
     __syncthreads();
     const int row = row_s, d = d_s;
     if (row < 0) return;
@@ -1471,7 +1480,7 @@ __global__ __launch_bounds__(256) void accept_pick_kernel(const float *__restric
     __shared__ double target_s;
     __shared__ Decision dec_s;
     __shared__ ExpEntry tab[16];
-    load_exp_tab(tab);
+    const ExpEntry entry = exp_entry();
     if (step_dev) step = *step_dev;
     if (threadIdx.x < 64) {
         // RC <= 64: lane c's chunk; the target's chunk is the last one whose
@@ -1493,6 +1502,7 @@ __global__ __launch_bounds__(256) void accept_pick_kernel(const float *__restric
             target_s = dec.target - (c ? run : 0.0);
         }
     }
+    put_exp_entry(tab, entry);
     __syncthreads();
     const Decision dec = dec_s;
     int next = dec.next;

@@ -299,3 +299,35 @@ def test_difference_past_the_float_range_has_no_weight(dev, stream, V):
     logits[:, 9] = 2.9e38
     for top_k, top_p in [(0, 1.0), (0, 0.9), (5, 1.0), (5, 0.9)]:
         assert _check_truncated(dev, stream, logits, np.array([9], np.int32), 1e38, top_k, top_p, 3, 1) == 0
+
+
+# More rows than CUs: workgroups of eight waves, with a shorter candidate list;
+# rows of up to its 6144 entries are cut in LDS, up to 8192 from memory. At
+# 2100 rows a row's area holds some 240 candidates: a flat distribution's
+# boundary bin and most top-k sets are gathered by the cut's workgroup, up to
+# the list's length, and longer ones cut over the whole row. Rising rows put
+# all their candidates next to each other.
+@pytest.mark.parametrize("B,k,V,shape,top_k,top_p", [
+    (257, 0, 6144, "normal", 0, 0.9), (300, 0, 6145, "normal", 50, 1.0), (300, 0, 8192, "normal", 0, 0.9),
+    (150, 1, 7001, "normal", 900, 0.9), (257, 0, 8193, "normal", 0, 0.9),
+    (2100, 0, 20011, "normal", 0, 0.9), (2100, 0, 20011, "normal", 3000, 1.0), (2100, 0, 20011, "normal", 300, 0.8),
+    (2100, 0, 20011, "normal", 6100, 0.95), (2100, 0, 20011, "normal", 7000, 1.0), (2100, 0, 20011, "rising", 0, 0.9),
+    (70, 8, 20011, "rising", 1000, 0.999), (20, 8, 20011, "rising", 4000, 0.9), (2100, 0, 20011, "equal", 0, 0.5)])
+def test_truncated_batches_match_oracle(dev, stream, B, k, V, shape, top_k, top_p):
+    rng = np.random.default_rng(B + V + top_k)
+    logits = rng.standard_normal((B, k + 1, V), np.float32)
+    if shape == "rising":
+        logits.sort(axis=-1)
+    if shape == "equal":
+        logits[:] = 0.25
+    drafts = logits[:, :k].argmax(2).astype(np.int32)
+    T = 1.0
+    p = hip.accept_params(hip.ACCEPT_STOCHASTIC, B, k, V, temperature=T, top_k=top_k, top_p=top_p, seed=8, step=2)
+    res, dbg = _run(dev, stream, logits, drafts, p)
+    for b in (0, B // 3, B - 1):
+        a, nxt, pd, ua = O.accept_stochastic(logits[b], drafts[b], T, 8, 2, b, top_k, top_p)
+        for i in range(min(a, int(res[b, 0])) + 1):
+            total = O.target_weights(logits[b, i], T, top_k, top_p)[2]
+            assert abs(dbg[b, i, 2] - total) <= 1e-12 * total
+            assert i == k or abs(dbg[b, i, 0] - pd[i]) <= 1e-9 * pd[i] + 1e-15
+        assert (int(res[b, 0]), int(res[b, 1])) == (a, nxt)

@@ -291,8 +291,14 @@ __global__ __launch_bounds__(256) void accept_weights_kernel(const float *__rest
 // each — so the 64 lanes of an LDS atomic met on the same few addresses
 // (95 us at 144 rows of 151936), and its boundary bucket still held 17
 // thousand members, for three more passes of one workgroup per row (136 us).)
-// Rows whose candidates do not fit (a bin of many equal logits, or a cut in
-// the open last bin) take the radix selection over the whole row.
+// Candidates without room in the row's area (thousands of rows leave each a
+// few KB; a sorted row puts all of them into one wave's segment) are gathered
+// once more by the row's workgroup, into its own list; before that such rows
+// took the radix selection over the whole row, four more passes (2500 rows of
+// 151936, T 1.5, top-p 0.9: 6.20 -> 3.13 ms, top-k 2000: 4.01 -> 2.39; 420
+// sorted rows of 27205, top-k 1000: 247 -> 135 us). That is left for rows
+// whose list is too short as well (a bin of many equal logits) or whose cut
+// lies in the open last bin.
 //
 // Scratch of one (request, row): C * kRowArea bytes of
 //   Moments [C]              per-chunk sums behind the bin width
@@ -301,7 +307,6 @@ __global__ __launch_bounds__(256) void accept_weights_kernel(const float *__rest
 //   Member [segs][seg]       the candidates
 constexpr int kBins = 1024;    // most bins of a histogram
 constexpr int kBinWaves = 8;   // waves of a bins workgroup, a histogram each
-constexpr int kCandMost = 8192;
 constexpr int kDirectMost = 8192;  // vocabulary whose rows go to LDS whole
 constexpr int kRankMost = 512;  // candidates ordered by counting
 
@@ -315,6 +320,7 @@ struct TruncGeo {
     int HC;    // histogram chunks of a row
     int KC;    // collecting chunks of a row (4 waves each)
     int seg;   // candidates of one collecting wave
+    int cap;   // candidates of a row
     uint32_t bins_off, cnt_off, cand_off;  // in the row's area
 };
 
@@ -328,10 +334,13 @@ struct RowCut {
     double before_rest;  // ... without the draft
     float best_v;        // row maximum
     int best_i;
-    int status;  // kCutFound: the candidates decide; kCutAll: nothing is cut; kCutRow: scan the row
-    int pad;
+    int status;
+    int bnd;      // (collect -> cut) the boundary bin
+    float scale;  // (collect -> cut) wave_bin_scale of the row
 };
-enum { kCutFound = 0, kCutAll = 1, kCutRow = 2 };
+// The candidates decide; nothing is cut; scan the row; the candidates decide
+// but have no room in the row's area.
+enum { kCutFound = 0, kCutAll = 1, kCutRow = 2, kCutGather = 3 };
 
 // A row's record lies at the end of its area.
 __device__ __forceinline__ RowCut &row_cut(uint8_t *area, const Geo &g, int b, int row) {
@@ -339,10 +348,11 @@ __device__ __forceinline__ RowCut &row_cut(uint8_t *area, const Geo &g, int b, i
 }
 
 // Bins per unit of logit below the maximum: the range down to three standard
-// deviations under the mean, or 48 T if that is less (the weights below it
-// are under 1e-20 of the largest), in NB steps. Every workgroup of a row
-// computes the same value (fixed order), so the bins of its passes agree.
-// Wave 0 of a workgroup.
+// deviations under the mean in NB steps; weighed bins (COUNT false) end at
+// 48 T if that is less (the weights below it are under 1e-20 of the largest).
+// Every workgroup of a row computes the same value (fixed order), so the bins
+// of its passes agree. Wave 0 of a workgroup.
+template <bool COUNT>
 __device__ __forceinline__ float wave_bin_scale(const Moments *__restrict__ m, int C, float mx, const Temp &t, int NB) {
     const int lane = threadIdx.x & 63;
     float n = 0.f, s1 = 0.f, s2 = 0.f;
@@ -360,7 +370,7 @@ __device__ __forceinline__ float wave_bin_scale(const Moments *__restrict__ m, i
     const float mean = s1 / n;
     const float sd = sqrtf(fmaxf(s2 / n - mean * mean, 1e-6f * mean * mean));
     float range = (mx - mean) + 3.f * sd;
-    if (!(range > 1e-30f && range < cap)) range = cap;
+    if (!(range > 1e-30f && range < (COUNT ? 1e30f : cap))) range = cap;
     return (float)NB / range;
 }
 
@@ -398,7 +408,7 @@ __global__ __launch_bounds__(64 * kBinWaves) void accept_bins_kernel(const float
     for (int i = threadIdx.x; i < kBinWaves * tg.NB; i += kT) hist[i] = (T)0;
     if (threadIdx.x < 64) {
         const Stat s = wave_best(stats + ((uint64_t)b * g.R + row) * g.C, g.C);
-        const float sc = wave_bin_scale(reinterpret_cast<const Moments *>(ra), g.C, s.v, t, tg.NB);
+        const float sc = wave_bin_scale<COUNT>(reinterpret_cast<const Moments *>(ra), g.C, s.v, t, tg.NB);
         if (threadIdx.x == 0) {
             mx_s = s.v;
             scale_s = sc;
@@ -463,7 +473,7 @@ __global__ __launch_bounds__(256) void accept_collect_kernel(const float *__rest
     __shared__ float mx_s, scale_s;
     __shared__ int best_i_s, bnd_s;
     __shared__ T wave_tot[4];
-    __shared__ T before_s;
+    __shared__ T before_s, upto_s;
     __shared__ ExpEntry tab[16];
     const ExpEntry entry = exp_entry();
     const int c = blockIdx.x, row = blockIdx.y, b = blockIdx.z;
@@ -483,13 +493,13 @@ __global__ __launch_bounds__(256) void accept_collect_kernel(const float *__rest
             if (i < per && lo + i < tg.NB) h[i] += hist[(uint64_t)ch * tg.NB + lo + i];
     if (threadIdx.x < 64) {
         const Stat s = wave_best(stats + ((uint64_t)b * g.R + row) * g.C, g.C);
-        const float sc = wave_bin_scale(reinterpret_cast<const Moments *>(ra), g.C, s.v, t, tg.NB);
+        const float sc = wave_bin_scale<COUNT>(reinterpret_cast<const Moments *>(ra), g.C, s.v, t, tg.NB);
         if (threadIdx.x == 0) {
             mx_s = s.v;
             scale_s = sc;
             best_i_s = s.i;
             bnd_s = tg.NB;
-            before_s = (T)0;
+            before_s = upto_s = (T)0;
         }
     }
     T sum = (T)0;
@@ -524,7 +534,7 @@ __global__ __launch_bounds__(256) void accept_collect_kernel(const float *__rest
     {
         T cum = exc;
         int pick = -1;
-        T before = (T)0;
+        T before = (T)0, upto = (T)0;
 #pragma unroll
         for (int i = 0; i < kPer; i++) {
             if (i >= per || lo + i >= tg.NB || pick >= 0) continue;
@@ -535,18 +545,23 @@ __global__ __launch_bounds__(256) void accept_collect_kernel(const float *__rest
             if (hit) {
                 pick = lo + i;
                 before = cum;
+                upto = next;
             }
             cum = next;
         }
         if (pick >= 0) atomicMin(&bnd_s, pick);
         __syncthreads();
-        if (pick >= 0 && bnd_s == pick) before_s = before;
+        if (pick >= 0 && bnd_s == pick) {
+            before_s = before;
+            upto_s = upto;
+        }
     }
     __syncthreads();
     const int bnd = bnd_s;
     int status = kCutFound;
     if (COUNT) {
-        if (tot <= (T)top_k || bnd >= tg.NB - 1) status = kCutRow;
+        if (tot <= (T)top_k || bnd >= tg.NB - 1 || upto_s > (T)tg.cap) status = kCutRow;
+        else if (upto_s > (T)(tg.KC * 4 * tg.seg)) status = kCutGather;
     } else {
         if (!(total > 0.0) || isinf(total) || bnd >= tg.NB) status = kCutAll;
         else if (bnd == tg.NB - 1) status = kCutRow;
@@ -562,6 +577,8 @@ __global__ __launch_bounds__(256) void accept_collect_kernel(const float *__rest
         o.best_v = mx;
         o.best_i = best_i_s;
         o.status = status;
+        o.bnd = bnd;
+        o.scale = scale;
     }
     const int w = c * 4 + wave;
     uint32_t found = 0u;
@@ -592,11 +609,17 @@ __global__ __launch_bounds__(256) void accept_collect_kernel(const float *__rest
 // over the 32-bit order key, histograms in LDS. Each wave fills its own
 // histogram and the waves are combined in wave order, so weight sums do not
 // depend on wave scheduling.
-constexpr int kSelWaves = 16;
+//
+// A workgroup of W waves: sixteen and a long candidate list while every row
+// can have a CU, else eight and a list that lets a CU hold two workgroups
+// (2160 rows of 8192, top-k 40: 202 -> 132 us; 1350 of 8200, top-k 1000: 139
+// -> 99; 2070 of 151936, T 1.5, top-p 0.9: 1.59 -> 1.45 ms).
+constexpr int cand_most(int W) { return W == 16 ? 8192 : 6144; }
 
+template <int W>
 struct SelShared {
-    uint32_t cnt[kSelWaves][256];
-    double wsum[kSelWaves][256];
+    uint32_t cnt[W][256];
+    double wsum[W][256];
     uint32_t tc[256];
     double tw[256];
     uint32_t prefix;    // digits chosen so far
@@ -620,9 +643,9 @@ struct SelSrc {
 };
 
 // f(logit, id) for every valid element, in a fixed order per thread.
-template <class F>
+template <int W, class F>
 __device__ __forceinline__ void for_each(const SelSrc &src, F f) {
-    constexpr int kStride = kSelWaves * 64;
+    constexpr int kStride = W * 64;
     if (src.list) {
         for (int i = threadIdx.x; i < src.n; i += kStride)
             if (valid_logit(src.list[i].l)) f(src.list[i].l, src.list[i].j);
@@ -642,28 +665,28 @@ __device__ __forceinline__ void for_each(const SelSrc &src, F f) {
 }
 
 // Histogram of the next digit over the elements that `sel` admits.
-template <bool W, class Sel>
-__device__ __forceinline__ void hist_pass(const SelSrc &src, float mx, const Temp &t, SelShared &s, int shift, Sel sel) {
+template <bool WEIGH, int W, class Sel>
+__device__ __forceinline__ void hist_pass(const SelSrc &src, float mx, const Temp &t, SelShared<W> &s, int shift, Sel sel) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for (int b = lane; b < 256; b += 64) {
         s.cnt[wave][b] = 0u;
-        if (W) s.wsum[wave][b] = 0.0;
+        if (WEIGH) s.wsum[wave][b] = 0.0;
     }
     __syncthreads();
-    for_each(src, [&](float l, int j) __attribute__((always_inline)) {
+    for_each<W>(src, [&](float l, int j) __attribute__((always_inline)) {
         const uint32_t k = order_key(l);
         if (!sel(k, j)) return;
         const int b = (k >> shift) & 255u;
         atomicAdd(&s.cnt[wave][b], 1u);
-        if (W) unsafeAtomicAdd(&s.wsum[wave][b], soft_weight(l, mx, t, s.tab));
+        if (WEIGH) unsafeAtomicAdd(&s.wsum[wave][b], soft_weight(l, mx, t, s.tab));
     });
     __syncthreads();
     if (threadIdx.x < 256) {
         uint32_t c = 0u;
         double w = 0.0;
-        for (int q = 0; q < kSelWaves; q++) {
+        for (int q = 0; q < W; q++) {
             c += s.cnt[q][threadIdx.x];
-            if (W) w += s.wsum[q][threadIdx.x];
+            if (WEIGH) w += s.wsum[q][threadIdx.x];
         }
         s.tc[threadIdx.x] = c;
         s.tw[threadIdx.x] = w;
@@ -678,7 +701,8 @@ __device__ __forceinline__ void hist_pass(const SelSrc &src, float mx, const Tem
 // lanes-before-it prefix (a fixed shuffle tree, so the sums are the same on
 // every run), then its own buckets in order; the first lane that reaches
 // the need picks. (One thread walking 256 LDS entries took ~16 us a pass.)
-__device__ __forceinline__ void scan_buckets(SelShared &s, bool descending, bool by_weight, uint32_t need_c,
+template <int W>
+__device__ __forceinline__ void scan_buckets(SelShared<W> &s, bool descending, bool by_weight, uint32_t need_c,
                                              double need_w, int shift) {
     const int lane = threadIdx.x & 63;
     uint32_t bc[4], lc = 0u;
@@ -733,7 +757,8 @@ __device__ __forceinline__ void scan_buckets(SelShared &s, bool descending, bool
 }
 
 // Wave 0: the sums of the 256 bucket counts and weights (fixed tree order).
-__device__ __forceinline__ void bucket_totals(const SelShared &s, uint32_t *c_out, double *w_out) {
+template <int W>
+__device__ __forceinline__ void bucket_totals(const SelShared<W> &s, uint32_t *c_out, double *w_out) {
     const int lane = threadIdx.x & 63;
     uint32_t c = 0u;
     double w = 0.0;
@@ -753,11 +778,12 @@ __device__ __forceinline__ void bucket_totals(const SelShared &s, uint32_t *c_ou
 
 // The need-th smallest id (1-based) among the elements with order key `key`
 // that lie inside `cut`.
-__device__ int select_id(const float *p, int V, SelShared &s, uint32_t key, Cut cut, uint32_t need) {
-    // One ordered sweep: 8 slices of kSelWaves * 64 consecutive ids per
+template <int W>
+__device__ int select_id(const float *p, int V, SelShared<W> &s, uint32_t key, Cut cut, uint32_t need) {
+    // One ordered sweep: 8 slices of W * 64 consecutive ids per
     // step, the matches of each wave counted by ballot, and the step where
     // the running count reaches `need` resolved by rank.
-    constexpr int kT = kSelWaves * 64, kU = 8;
+    constexpr int kT = W * 64, kU = 8;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     if (threadIdx.x == 0) s.id = INT_MAX;
     uint32_t before = 0u;
@@ -779,16 +805,16 @@ __device__ int select_id(const float *p, int V, SelShared &s, uint32_t key, Cut 
         }
         __syncthreads();
         uint32_t tot = 0u;
-        for (int q = 0; q < kU * kSelWaves; q++) tot += s.cnt[q / kSelWaves][q % kSelWaves];
+        for (int q = 0; q < kU * W; q++) tot += s.cnt[q / W][q % W];
         if (before + tot >= need) {
             uint32_t r = before;
 #pragma unroll
             for (int u = 0; u < kU; u++) {
                 uint32_t pw = 0u;
-                for (int q = 0; q < kSelWaves; q++) pw += q < wave ? s.cnt[u][q] : 0u;
+                for (int q = 0; q < W; q++) pw += q < wave ? s.cnt[u][q] : 0u;
                 const uint32_t rank = r + pw + (uint32_t)__popcll(bal[u] & ((1ull << lane) - 1ull)) + 1u;
                 if (m[u] && rank == need) s.id = base + u * kT + threadIdx.x;
-                for (int q = 0; q < kSelWaves; q++) r += s.cnt[u][q];
+                for (int q = 0; q < W; q++) r += s.cnt[u][q];
             }
             break;
         }
@@ -815,7 +841,8 @@ __device__ __forceinline__ uint32_t tie_members(double before, double w, double 
 
 // The cut of one row by radix selection over src. With `tail` (candidates of
 // one bin): the weight `before` lies ahead of src's elements, of `total`.
-__device__ __forceinline__ Cut radix_cut(const SelSrc src, SelShared &s, float mx, const Temp t, int top_k, float top_p,
+template <int W>
+__device__ __forceinline__ Cut radix_cut(const SelSrc src, SelShared<W> &s, float mx, const Temp t, int top_k, float top_p,
                                          bool tail, double before, double total) {
     Cut cut{0u, INT_MAX};
     // top-k: the top_k-th element in (logit desc, id asc) order (sampling.go:90-92).
@@ -911,22 +938,82 @@ __device__ __forceinline__ Cut radix_cut(const SelSrc src, SelShared &s, float m
 }
 
 // Sum over the workgroup in wave order, in every thread.
+template <int W>
 __device__ __forceinline__ double block_sum(double v, double *waves) {
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
     __syncthreads();
     if ((threadIdx.x & 63) == 0) waves[threadIdx.x >> 6] = v;
     __syncthreads();
     double t = 0.0;
-    for (int w = 0; w < kSelWaves; w++) t += waves[w];
+    for (int w = 0; w < W; w++) t += waves[w];
     return t;
+}
+
+// A row's candidates (see accept_collect_kernel) side by side in the list, by
+// one workgroup: each wave fills a segment in (iteration, lane) order, then
+// the segments close up. Returns their number, or -1 if a segment is too
+// short. Waves take every sixteenth 64 ids, so a run of large logits spreads
+// over them.
+template <int W>
+__device__ __forceinline__ int gather(const float *__restrict__ p, int V, const RowCut &in, int NB, bool above,
+                                      Member *list, uint32_t *found_s) {
+    constexpr int kT = 64 * W, kSeg = cand_most(W) / W, kPer = cand_most(W) / kT, kU = 8;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    uint32_t found = 0u;
+    for (int j0 = threadIdx.x; j0 - (int)threadIdx.x < V && found <= (uint32_t)kSeg; j0 += kU * kT) {
+        float l[kU];
+#pragma unroll
+        for (int u = 0; u < kU; u++) l[u] = j0 + kT * u < V ? p[j0 + kT * u] : NAN;
+#pragma unroll
+        for (int u = 0; u < kU; u++) {
+            const int bin = bin_of(l[u], in.best_v, in.scale, NB);
+            const bool take = valid_logit(l[u]) && (above ? bin <= in.bnd : bin == in.bnd);
+            const uint64_t m = __ballot(take);
+            const uint32_t at = found + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+            if (take && at < (uint32_t)kSeg) list[wave * kSeg + at] = Member{l[u], j0 + kT * u};
+            found += (uint32_t)__popcll(m);
+        }
+    }
+    if (lane == 0) found_s[wave] = found;
+    __syncthreads();
+    uint32_t at[W + 1];
+    at[0] = 0u;
+    bool ok = true;
+#pragma unroll
+    for (int q = 0; q < W; q++) {
+        ok = ok && found_s[q] <= (uint32_t)kSeg;
+        at[q + 1] = at[q] + found_s[q];
+    }
+    const int n = (int)at[W];
+    Member m[kPer];
+#pragma unroll
+    for (int u = 0; u < kPer; u++) {
+        const uint32_t i = threadIdx.x + u * kT;
+        if (!ok || i >= (uint32_t)n) continue;
+        uint32_t from = 0u;
+#pragma unroll
+        for (int q = 0; q < W; q++)
+            if (i >= at[q]) from = q * kSeg + i - at[q];
+        m[u] = list[from];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kPer; u++) {
+        const uint32_t i = threadIdx.x + u * kT;
+        if (ok && i < (uint32_t)n) list[i] = m[u];
+    }
+    __syncthreads();
+    return ok ? n : -1;
 }
 
 // One workgroup per row: the exact cut, and the kept weight without the
 // draft and of the draft. Up to kRankMost candidates are put in order by
-// counting (thread i counts what lies ahead of candidate i); more take the
-// radix selection. `direct`: no candidates were collected, the row itself is
-// taken (into LDS).
-__global__ __launch_bounds__(64 * kSelWaves) void accept_cut_kernel(const float *__restrict__ logits, Geo g, TruncGeo tg,
+// counting (thread i counts what lies ahead of candidate i) and their weights
+// summed in that order (some 450 candidates of one row: 63 us a call; with the
+// sums taken in the counting loop 82); more take the radix selection. `direct`: no candidates were collected, the row itself is
+// taken (1: into LDS).
+template <int W>
+__global__ __launch_bounds__(64 * W, 4) void accept_cut_kernel(const float *__restrict__ logits, Geo g, TruncGeo tg,
                                                                     const int32_t *__restrict__ drafts,
                                                                     const Stat *__restrict__ stats, int top_k, float top_p,
                                                                     Temp t, uint8_t *__restrict__ area, int direct) {
@@ -934,8 +1021,8 @@ __global__ __launch_bounds__(64 * kSelWaves) void accept_cut_kernel(const float 
     const float *p = row_ptr(logits, g, b, row);
     uint8_t *ra = row_area(area, g, b, row);
     RowCut &rc = row_cut(area, g, b, row);
-    __shared__ SelShared s;
-    __shared__ double waves[kSelWaves];
+    __shared__ SelShared<W> s;
+    __shared__ double waves[W];
     __shared__ uint32_t seg_at[260];
     __shared__ int n_s, end_s, last_s;
     extern __shared__ __attribute__((aligned(16))) uint8_t cut_dyn[];
@@ -944,7 +1031,8 @@ __global__ __launch_bounds__(64 * kSelWaves) void accept_cut_kernel(const float 
     const ExpEntry entry = exp_entry();
     if (direct) {
         __shared__ Stat best_s;
-        for (int j = threadIdx.x; j < g.V; j += 64 * kSelWaves) list[j] = Member{p[j], j};
+        if (direct == 1)
+            for (int j = threadIdx.x; j < g.V; j += 64 * W) list[j] = Member{p[j], j};
         if (threadIdx.x < 64) {
             const Stat best = wave_best(stats + ((uint64_t)b * g.R + row) * g.C, g.C);
             if (threadIdx.x == 0) best_s = best;
@@ -986,20 +1074,24 @@ __global__ __launch_bounds__(64 * kSelWaves) void accept_cut_kernel(const float 
             }
             if (threadIdx.x == 63) seg_at[256] = at;
             const uint64_t good = __ballot(ok);
-            if (threadIdx.x == 63) n_s = good == ~0ull && at <= (uint32_t)kCandMost ? (int)at : -1;
+            if (threadIdx.x == 63) n_s = good == ~0ull && at <= (uint32_t)cand_most(W) ? (int)at : -1;
         }
         __syncthreads();
         fits = n_s >= 0;
     }
     if (fits) {
         const Member *src = reinterpret_cast<const Member *>(ra + tg.cand_off);
-        for (int q = threadIdx.x >> 6; q < segs; q += kSelWaves) {
+        for (int q = threadIdx.x >> 6; q < segs; q += W) {
             const uint32_t a = seg_at[q], n = seg_at[q + 1] - a;
             for (uint32_t i = threadIdx.x & 63; i < n; i += 64) list[a + i] = src[(uint64_t)q * tg.seg + i];
         }
         __syncthreads();
     }
-    const int n = fits ? n_s : 0;
+    int n = fits ? n_s : 0;
+    if (!fits && (in.status == kCutFound || in.status == kCutGather)) {
+        n = gather<W>(p, g.V, in, tg.NB, top_k > 0, list, seg_at);
+        fits = n >= 0;
+    }
     Cut cut{0u, INT_MAX};
     if (fits && n <= kRankMost) {
         // composite order: a larger (key, ~id) is ahead
@@ -1037,7 +1129,7 @@ __global__ __launch_bounds__(64 * kSelWaves) void accept_cut_kernel(const float 
             if (lane == 63) waves[wave] = inc;
             __syncthreads();
             sum = 0.0;
-            for (int q = 0; q < kSelWaves; q++) {
+            for (int q = 0; q < W; q++) {
                 if (q == wave) base = sum;
                 sum += waves[q];
             }
@@ -1061,17 +1153,17 @@ __global__ __launch_bounds__(64 * kSelWaves) void accept_cut_kernel(const float 
         const unsigned long long last = sorted[last_s];
         cut = Cut{(uint32_t)(last >> 32), (int32_t)~(uint32_t)last};
     } else {
-        const SelSrc src{p, g.V, fits || direct ? list : nullptr, fits ? n : g.V, fits && top_k > 0};
+        const SelSrc src{p, g.V, fits || direct == 1 ? list : nullptr, fits ? n : g.V, fits && top_k > 0};
         cut = radix_cut(src, s, mx, t, top_k, top_p, fits && top_k <= 0, in.before, in.total);
         __syncthreads();
     }
     // the kept weight: candidates (after the bins above them), or the row
-    const SelSrc src{p, g.V, fits || direct ? list : nullptr, fits ? n : g.V, false};
+    const SelSrc src{p, g.V, fits || direct == 1 ? list : nullptr, fits ? n : g.V, false};
     double sum = 0.0;
-    for_each(src, [&](float l, int j) __attribute__((always_inline)) {
+    for_each<W>(src, [&](float l, int j) __attribute__((always_inline)) {
         if (j != d && in_cut(order_key(l), j, cut)) sum += soft_weight(l, mx, t, s.tab);
     });
-    sum = block_sum(sum, waves);
+    sum = block_sum<W>(sum, waves);
     if (threadIdx.x == 0) {
         rc.best_v = in.best_v;
         rc.best_i = in.best_i;
@@ -1541,6 +1633,9 @@ Geo make_geo(const yuuka_accept_params &p) {
     return g;
 }
 
+// Waves of a cut workgroup (see SelShared).
+int cut_waves(int rows) { return rows <= 256 ? 16 : 8; }
+
 // The layout of a row's area. The bins take at most about half of it, the
 // candidates the rest; few rows have many chunks and much room, thousands of
 // rows little (fewer bins, and more of their rows scan the row).
@@ -1555,7 +1650,8 @@ TruncGeo trunc_geo(const Geo &g) {
     t.cnt_off = t.bins_off + (uint32_t)(t.HC * t.NB * 8);
     t.cand_off = t.cnt_off + (uint32_t)(t.KC * 4 * 4);
     // (segments fill unevenly: twice the list's room where there is space)
-    t.seg = std::min((int)((bytes - t.cand_off) / sizeof(Member)), 2 * kCandMost) / (t.KC * 4);
+    t.cap = cand_most(cut_waves(rows));
+    t.seg = std::min((int)((bytes - t.cand_off) / sizeof(Member)), 2 * t.cap) / (t.KC * 4);
     return t;
 }
 
@@ -1616,17 +1712,19 @@ hipError_t launch_verify_accept(const float *logits, const int32_t *drafts, int3
     const uint32_t bins_lds = (uint32_t)(kBinWaves * tg.NB) * (top_k_on ? 4u : 8u);
     static bool attr = false;
     if (!attr) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(accept_cut_kernel),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, kCandMost * (int)sizeof(Member));
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(accept_cut_kernel<16>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, cand_most(16) * (int)sizeof(Member));
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(accept_cut_kernel<8>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, cand_most(8) * (int)sizeof(Member));
         (void)hipFuncSetAttribute(reinterpret_cast<const void *>(accept_bins_kernel<false>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, kBinWaves * kBins * 8);
         attr = true;
     }
-    int cand = std::min(kCandMost, tg.KC * 4 * tg.seg);
-    const int direct = (int)p.vocab <= kDirectMost ? 1 : 0;
+    int cand = tg.cap;
+    const int direct = (int)p.vocab <= kDirectMost ? (g.V <= tg.cap ? 1 : 2) : 0;
     if (direct) {
         accept_stats_kernel<false><<<sgrid, 256, 0, stream>>>(logits, g, stats, vec, wpc, nullptr);
-        cand = g.V;
+        cand = direct == 1 ? g.V : 0;
     } else if (top_k_on) {
         accept_stats_kernel<true><<<sgrid, 256, 0, stream>>>(logits, g, stats, vec, wpc, area);
         accept_bins_kernel<true><<<hgrid, 64 * kBinWaves, bins_lds, stream>>>(logits, g, tg, drafts, stats, t, area);
@@ -1636,8 +1734,11 @@ hipError_t launch_verify_accept(const float *logits, const int32_t *drafts, int3
         accept_bins_kernel<false><<<hgrid, 64 * kBinWaves, bins_lds, stream>>>(logits, g, tg, drafts, stats, t, area);
         accept_collect_kernel<false><<<kgrid, 256, 0, stream>>>(logits, g, tg, drafts, stats, tk, tp, t, area);
     }
-    accept_cut_kernel<<<rgrid, 64 * kSelWaves, (uint32_t)cand * sizeof(Member), stream>>>(logits, g, tg, drafts, stats, tk,
-                                                                                         tp, t, area, direct);
+    const uint32_t cut_lds = (uint32_t)cand * sizeof(Member);
+    if (cut_waves(g.B * g.R) == 16)
+        accept_cut_kernel<16><<<rgrid, 64 * 16, cut_lds, stream>>>(logits, g, tg, drafts, stats, tk, tp, t, area, direct);
+    else
+        accept_cut_kernel<8><<<rgrid, 64 * 8, cut_lds, stream>>>(logits, g, tg, drafts, stats, tk, tp, t, area, direct);
     // chunks of the drawn row: at most 64 (one per lane of pick), and their
     // sums fit the per-chunk sums' place
     const int RC = std::min(64, g.R * g.C);

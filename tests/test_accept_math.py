@@ -53,6 +53,31 @@ int main() {
     printf("overflow %d %d %d\n", exp_nonpos(exponent_of(-big, big, make_temp(1e38f)), kExpTab) == 0.0,
            exp_nonpos(exponent_of(-big, big, make_temp(1e-45f)), kExpTab) == 0.0,
            std::isnan(exp_nonpos(exponent_of(-big, big, make_temp(INFINITY)), kExpTab)));
+    // tie groups against one addition after the other
+    bad = 0;
+    long longest = 0;
+    for (int i = 0; i < 60000; i++) {
+        uint32_t ties = 1 + (uint32_t)std::exp(uniform(0, i % 100 ? 7 : 12));
+        double w = i % 3 ? std::exp(-uniform(0, 12)) : 1.0, before = i % 2 ? 0.0 : uniform(0, 2) * w * ties;
+        double total = (before + w * ties) * (i % 5 ? 1 + uniform(0, 1) : 1.0), p = (float)uniform(0.01, 1);
+        if (i % 7 == 0) p = 0.25 * (1 + i % 3);
+        if (i % 11 == 0) total = std::exp2(std::ceil(std::log2(total)));
+        // shares halfway between two multiples of a sum's last place
+        if (i % 13 == 0) w = std::ldexp(2 * (double)(rng() % 1000) + 1, -(int)(50 + rng() % 6)), total = 1.0, before = uniform(0, 1);
+        if (i % 17 == 0) w *= 1e-17;
+        uint32_t want = ties;
+        double cum = before / total;
+        for (uint32_t k = 1; k < ties; k++) {
+            cum += w / total;
+            if (cum >= p) {
+                want = k;
+                break;
+            }
+        }
+        if (tie_members(before, w, total, p, ties) != want) bad++;
+        if (want < ties && want > longest) longest = want;
+    }
+    printf("ties %ld %ld\n", bad, longest);
     printf("flat %d\n", exp_nonpos(exponent_of(-big, 0.f, make_temp(INFINITY)), kExpTab) == 1.0);
 }
 """
@@ -84,3 +109,7 @@ def test_exponent_is_the_correctly_rounded_quotient(report):
 
 def test_overflowed_differences_weigh_nothing(report):
     assert report["overflow"] == ["1", "1", "1"] and report["flat"] == ["1"]
+
+
+def test_tie_group_as_one_addition_after_the_other(report):
+    assert report["ties"][0] == "0" and int(report["ties"][1]) > 50000

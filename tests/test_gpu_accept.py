@@ -229,7 +229,8 @@ def test_truncation_tie_group_spanning_late_id_steps(dev, stream):
     (40001, "narrow", 0, 0.6, 1.0), (40001, "normal", 511, 1.0, 0.8), (40001, "normal", 6000, 0.999, 1.3),
     (40001, "sorted", 200, 0.95, 1.0), (40001, "sorted", 0, 0.95, 1.0), (20000, "equal", 0, 0.5, 1.0),
     (20000, "equal", 300, 0.5, 1.0), (40001, "masked", 40, 0.9, 0.7), (40001, "masked", 0, 0.999, 1.0),
-    (40001, "outlier", 0, 0.9, 1.0), (300, "normal", 20, 0.9, 0.7)])
+    (40001, "outlier", 0, 0.9, 1.0), (300, "normal", 20, 0.9, 0.7), (40001, "two", 0, 0.3, 1.0),
+    (40001, "two", 5000, 0.9, 1.3), (40001, "two", 0, 0.99, 1.0), (5000, "equal", 0, 0.7, 1.0), (5000, "two", 900, 0.8, 1.0)])
 def test_truncation_paths_match_oracle(dev, stream, V, shape, top_k, top_p, T):
     rng = np.random.default_rng(V + top_k)
     k = 3
@@ -238,6 +239,8 @@ def test_truncation_paths_match_oracle(dev, stream, V, shape, top_k, top_p, T):
         logits = -np.sort(-logits, axis=1)
     if shape == "equal":
         logits[:] = 0.25
+    if shape == "two":
+        logits = (logits > 2).astype(np.float32) * 3
     if shape == "masked":
         logits[rng.random(logits.shape) < 0.98] = -np.inf
     if shape == "outlier":

@@ -677,8 +677,18 @@ __device__ __forceinline__ void hist_pass(const SelSrc &src, float mx, const Tem
         const uint32_t k = order_key(l);
         if (!sel(k, j)) return;
         const int b = (k >> shift) & 255u;
-        atomicAdd(&s.cnt[wave][b], 1u);
-        if (WEIGH) unsafeAtomicAdd(&s.wsum[wave][b], soft_weight(l, mx, t, s.tab));
+        const double w = WEIGH ? soft_weight(l, mx, t, s.tab) : 0.0;
+        auto add = [&](uint32_t n) __attribute__((always_inline)) {
+            atomicAdd(&s.cnt[wave][b], n);
+            if (WEIGH) unsafeAtomicAdd(&s.wsum[wave][b], (double)n * w);
+        };
+        // the lanes that share the first one's key add once (64 adds to one
+        // address, one after the other, are what a row of equal logits costs
+        // otherwise)
+        const bool same = k == (uint32_t)__builtin_amdgcn_readfirstlane((int)k);
+        const uint64_t m = __ballot(same);
+        if (!same) add(1u);
+        else if (lane == __ffsll((unsigned long long)m) - 1) add((uint32_t)__popcll(m));
     });
     __syncthreads();
     if (threadIdx.x < 256) {
@@ -825,18 +835,6 @@ __device__ int select_id(const float *p, int V, SelShared<W> &s, uint32_t key, C
     const int id = s.id;
     __syncthreads();  // every thread has read the result before the state is reused
     return id;
-}
-
-// Members of a boundary tie group (weight w each) that top_p keeps: they join
-// one by one, as the sampler's running sum adds their shares
-// (sampling.go:107-113), from the weight `before` ahead of the group.
-__device__ __forceinline__ uint32_t tie_members(double before, double w, double total, double top_p, uint32_t ties) {
-    double cum = before / total;
-    for (uint32_t i = 1; i < ties; i++) {
-        cum += w / total;
-        if (cum >= top_p) return i;
-    }
-    return ties;
 }
 
 // The cut of one row by radix selection over src. With `tail` (candidates of

@@ -220,17 +220,21 @@ def test_truncation_tie_group_spanning_late_id_steps(dev, stream):
             assert _check_truncated(dev, stream, logits, drafts, 1.0, top_k, top_p, 21, step) == 0
 
 
-# Rows up to 8192 logits are cut in LDS whole; longer ones through the binned
-# candidates: by counting up to 512, by radix selection above, over the whole
-# row where the candidates do not fit (a sorted row fills one wave's segment,
-# equal logits one bin, a masked row ends in the open last bin).
+# Rows up to 8192 logits are cut in LDS whole, up to 16384 with top-k alone from
+# memory; longer ones through the binned candidates: by counting up to 512, by
+# radix selection above, over the whole row where the candidates do not fit
+# (equal logits fill one bin) or the cut is in the open last bin. A sorted row
+# fills one wave's segment; a masked row may have fewer valid logits than top-k.
 @pytest.mark.parametrize("V,shape,top_k,top_p,T", [
     (8192, "normal", 0, 0.9, 0.7), (8193, "normal", 0, 0.9, 0.7), (8193, "normal", 513, 0.97, 1.0),
     (40001, "narrow", 0, 0.6, 1.0), (40001, "normal", 511, 1.0, 0.8), (40001, "normal", 6000, 0.999, 1.3),
     (40001, "sorted", 200, 0.95, 1.0), (40001, "sorted", 0, 0.95, 1.0), (20000, "equal", 0, 0.5, 1.0),
     (20000, "equal", 300, 0.5, 1.0), (40001, "masked", 40, 0.9, 0.7), (40001, "masked", 0, 0.999, 1.0),
     (40001, "outlier", 0, 0.9, 1.0), (300, "normal", 20, 0.9, 0.7), (40001, "two", 0, 0.3, 1.0),
-    (40001, "two", 5000, 0.9, 1.3), (40001, "two", 0, 0.99, 1.0), (5000, "equal", 0, 0.7, 1.0), (5000, "two", 900, 0.8, 1.0)])
+    (40001, "two", 5000, 0.9, 1.3), (40001, "two", 0, 0.99, 1.0), (5000, "equal", 0, 0.7, 1.0), (5000, "two", 900, 0.8, 1.0),
+    (8193, "normal", 700, 1.0, 1.0), (16384, "normal", 40, 1.0, 0.7), (16384, "equal", 33, 1.0, 1.0),
+    (16385, "normal", 40, 1.0, 0.7), (12000, "masked", 5000, 1.0, 1.0), (40001, "masked", 6000, 1.0, 0.7),
+    (40001, "masked", 6000, 0.8, 0.7)])
 def test_truncation_paths_match_oracle(dev, stream, V, shape, top_k, top_p, T):
     rng = np.random.default_rng(V + top_k)
     k = 3

@@ -307,7 +307,14 @@ __global__ __launch_bounds__(256) void accept_weights_kernel(const float *__rest
 //   Member [segs][seg]       the candidates
 constexpr int kBins = 1024;    // most bins of a histogram
 constexpr int kBinWaves = 8;   // waves of a bins workgroup, a histogram each
-constexpr int kDirectMost = 8192;  // vocabulary whose rows go to LDS whole
+// Rows cut without bins: up to kDirectMost logits (in LDS where they fit the
+// list, see SelShared), and with top-k alone and a CU for every row up to
+// kDirectTopK, from memory (us, from memory / through the bins: 8200 logits,
+// top-k 40 34 / 37 at 1 row, 35 / 39 at 144 rows, top-k 1000 34 / 43 and 36 /
+// 45; 16000, top-k 40 38 / 37 and 41 / 42, top-k 1000 41 / 44 and 45 / 49;
+// 26307, top-k 40 48 / 38, 60 / 54).
+constexpr int kDirectMost = 8192;
+constexpr int kDirectTopK = 16384;
 constexpr int kRankMost = 512;  // candidates ordered by counting
 
 struct Member {
@@ -339,8 +346,8 @@ struct RowCut {
     float scale;  // (collect -> cut) wave_bin_scale of the row
 };
 // The candidates decide; nothing is cut; scan the row; the candidates decide
-// but have no room in the row's area.
-enum { kCutFound = 0, kCutAll = 1, kCutRow = 2, kCutGather = 3 };
+// but have no room in the row's area; top-k keeps every valid logit.
+enum { kCutFound = 0, kCutAll = 1, kCutRow = 2, kCutGather = 3, kCutNoTopK = 4 };
 
 // A row's record lies at the end of its area.
 __device__ __forceinline__ RowCut &row_cut(uint8_t *area, const Geo &g, int b, int row) {
@@ -560,7 +567,8 @@ __global__ __launch_bounds__(256) void accept_collect_kernel(const float *__rest
     const int bnd = bnd_s;
     int status = kCutFound;
     if (COUNT) {
-        if (tot <= (T)top_k || bnd >= tg.NB - 1 || upto_s > (T)tg.cap) status = kCutRow;
+        if (tot <= (T)top_k) status = kCutNoTopK;
+        else if (bnd >= tg.NB - 1 || upto_s > (T)tg.cap) status = kCutRow;
         else if (upto_s > (T)(tg.KC * 4 * tg.seg)) status = kCutGather;
     } else {
         if (!(total > 0.0) || isinf(total) || bnd >= tg.NB) status = kCutAll;
@@ -1152,7 +1160,7 @@ __global__ __launch_bounds__(64 * W, 4) void accept_cut_kernel(const float *__re
         cut = Cut{(uint32_t)(last >> 32), (int32_t)~(uint32_t)last};
     } else {
         const SelSrc src{p, g.V, fits || direct == 1 ? list : nullptr, fits ? n : g.V, fits && top_k > 0};
-        cut = radix_cut(src, s, mx, t, top_k, top_p, fits && top_k <= 0, in.before, in.total);
+        cut = radix_cut(src, s, mx, t, in.status == kCutNoTopK ? 0 : top_k, top_p, fits && top_k <= 0, in.before, in.total);
         __syncthreads();
     }
     // the kept weight: candidates (after the bins above them), or the row
@@ -1634,15 +1642,17 @@ Geo make_geo(const yuuka_accept_params &p) {
 // Waves of a cut workgroup (see SelShared).
 int cut_waves(int rows) { return rows <= 256 ? 16 : 8; }
 
-// The layout of a row's area. The bins take at most about half of it, the
+// The layout of a row's area. A chunk has a few thousand logits, or the
+// workgroups do little but add up the histograms (20 rows of 8200..32000,
+// top-p 0.9, with up to 52 chunks of a row: 56 us; now 39..43). The bins take at most about half of it, the
 // candidates the rest; few rows have many chunks and much room, thousands of
 // rows little (fewer bins, and more of their rows scan the row).
 TruncGeo trunc_geo(const Geo &g) {
     TruncGeo t;
     const int rows = g.B * g.R;
     t.NB = g.C >= 8 ? kBins : (g.C >= 4 ? 512 : (g.C >= 2 ? 256 : 128));
-    t.HC = std::max(1, std::min(16, g.C / 5));
-    t.KC = std::max(1, std::min(std::min(64, g.C), (1024 + rows - 1) / rows));
+    t.HC = std::max(1, std::min({16, g.C / 5, g.V / 8192}));
+    t.KC = std::max(1, std::min({64, g.C, (1024 + rows - 1) / rows, g.V / 4096}));
     const uint32_t bytes = (uint32_t)((uint64_t)g.C * kRowArea - sizeof(RowCut));
     t.bins_off = (uint32_t)(g.C * sizeof(Moments));
     t.cnt_off = t.bins_off + (uint32_t)(t.HC * t.NB * 8);
@@ -1719,7 +1729,7 @@ hipError_t launch_verify_accept(const float *logits, const int32_t *drafts, int3
         attr = true;
     }
     int cand = tg.cap;
-    const int direct = (int)p.vocab <= kDirectMost ? (g.V <= tg.cap ? 1 : 2) : 0;
+    const int direct = (int)p.vocab <= kDirectMost ? (g.V <= tg.cap ? 1 : 2) : (top_k_on && !top_p_on && g.V <= kDirectTopK && g.B * g.R <= 256 ? 2 : 0);
     if (direct) {
         accept_stats_kernel<false><<<sgrid, 256, 0, stream>>>(logits, g, stats, vec, wpc, nullptr);
         cand = direct == 1 ? g.V : 0;

@@ -1668,8 +1668,8 @@ TruncGeo trunc_geo(const Geo &g) {
 uint64_t accept_scratch_bytes(const yuuka_accept_params &p) {
     const Geo g = make_geo(p);
     const uint64_t n = (uint64_t)g.B * g.R * g.C;
-    return ((n * sizeof(Stat) + 255) & ~255ull) + n * sizeof(double) +
-           (uint64_t)g.B * g.R * (sizeof(double) + sizeof(Cut)) + 256 + n * kRowArea;
+    return ((n * sizeof(Stat) + 255) & ~255ull) + n * sizeof(double) + (uint64_t)g.B * g.R * sizeof(double) + 256 +
+           n * kRowArea;
 }
 
 hipError_t launch_router_normal(float *logits, int rows, int E, uint64_t seed, uint32_t layer, const uint64_t *step,

@@ -269,6 +269,11 @@ def test_fused_gemm_few_row_edges(dev, stream, segs, k, rows, norm):
         bound = _rounding_bound(dt, w, n, k, y)
         assert np.all(np.abs(gv - want) <= bound + 1e-30)
         assert np.all(gv[rows // 2] == 0.0)
+        # the bound by norms is some 5 % of a typical output at these K: it
+        # finds a wrong index, MANY_BUDGET on the ordinary rows lost precision
+        if n > 1:
+            rest = [r for r in range(1, rows) if r != rows // 2]
+            _check(gv[rest], want[rest], budget=MANY_BUDGET)
 
 
 @pytest.mark.parametrize("n,k,rows", [(7, 256, 9), (2049, 768, 16), (2560, 2560, 30), (5001, 512, 48)])
@@ -281,10 +286,13 @@ def test_fused_gemm_few_row_swiglu_edges(dev, stream, n, k, rows):
     y = O.rmsnorm_rows(x, g, 1e-6)
     gate, up = (_want(O.Q4_K, w, n, k, y).astype(np.float64) for w in (wg, wu))
     silu = gate / (1 + np.exp(-np.clip(gate, -700, 700)))
-    # either product's rounding as above, through SiLU (slope at most 1.1) and
-    # the product
-    eg, eu = (_rounding_bound(O.Q4_K, w, n, k, y) for w in (wg, wu))
-    assert np.all(np.abs(got - silu * up) <= 1.1 * eg * np.abs(up) + np.abs(silu) * eu + 1.1 * eg * eu + 1e-30)
+    # either product's rounding as above, and MANY_BUDGET of its rms, through
+    # SiLU (slope at most 1.1) and the product (whose largest values are many
+    # times its rms, so a share of that is no bound of theirs)
+    err = np.abs(got - silu * up)
+    for eg, eu in ([_rounding_bound(O.Q4_K, w, n, k, y) for w in (wg, wu)],
+                   [MANY_BUDGET * np.sqrt(np.mean(v ** 2)) for v in (gate, up)]):
+        assert np.all(err <= 1.1 * eg * np.abs(up) + np.abs(silu) * eu + 1.1 * eg * eu + 1e-30)
 
 
 def test_fused_gemm_many_rows_epilogues(dev, stream):

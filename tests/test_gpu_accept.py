@@ -225,6 +225,8 @@ def test_truncation_tie_group_spanning_late_id_steps(dev, stream):
 # radix selection above, over the whole row where the candidates do not fit
 # (equal logits fill one bin) or the cut is in the open last bin. A sorted row
 # fills one wave's segment; a masked row may have fewer valid logits than top-k.
+# More than 8192 of top-k are cut among the boundary bin's members, and a
+# selection over the row lists a bucket's members once they are few enough.
 @pytest.mark.parametrize("V,shape,top_k,top_p,T", [
     (8192, "normal", 0, 0.9, 0.7), (8193, "normal", 0, 0.9, 0.7), (8193, "normal", 513, 0.97, 1.0),
     (40001, "narrow", 0, 0.6, 1.0), (40001, "normal", 511, 1.0, 0.8), (40001, "normal", 6000, 0.999, 1.3),
@@ -234,7 +236,9 @@ def test_truncation_tie_group_spanning_late_id_steps(dev, stream):
     (40001, "two", 5000, 0.9, 1.3), (40001, "two", 0, 0.99, 1.0), (5000, "equal", 0, 0.7, 1.0), (5000, "two", 900, 0.8, 1.0),
     (8193, "normal", 700, 1.0, 1.0), (16384, "normal", 40, 1.0, 0.7), (16384, "equal", 33, 1.0, 1.0),
     (16385, "normal", 40, 1.0, 0.7), (12000, "masked", 5000, 1.0, 1.0), (40001, "masked", 6000, 1.0, 0.7),
-    (40001, "masked", 6000, 0.8, 0.7)])
+    (40001, "masked", 6000, 0.8, 0.7), (40001, "normal", 9000, 1.0, 1.0), (40001, "normal", 20000, 0.9, 1.3),
+    (40001, "coarse", 9001, 1.0, 1.0), (40001, "coarse", 9001, 0.95, 1.3), (40001, "coarse", 0, 0.97, 1.3),
+    (40001, "outlier", 200, 1.0, 1.0), (40001, "outlier", 9000, 0.9, 5e3), (40001, "outlier", 0, 0.99, 5e3)])
 def test_truncation_paths_match_oracle(dev, stream, V, shape, top_k, top_p, T):
     rng = np.random.default_rng(V + top_k)
     k = 3
@@ -243,6 +247,8 @@ def test_truncation_paths_match_oracle(dev, stream, V, shape, top_k, top_p, T):
         logits = -np.sort(-logits, axis=1)
     if shape == "equal":
         logits[:] = 0.25
+    if shape == "coarse":
+        logits = (np.round(logits * 20) / 20).astype(np.float32)
     if shape == "two":
         logits = (logits > 2).astype(np.float32) * 3
     if shape == "masked":

@@ -298,7 +298,8 @@ __global__ __launch_bounds__(256) void accept_weights_kernel(const float *__rest
 // 151936, T 1.5, top-p 0.9: 6.20 -> 3.13 ms, top-k 2000: 4.01 -> 2.39; 420
 // sorted rows of 27205, top-k 1000: 247 -> 135 us). That is left for rows
 // whose list is too short as well (a bin of many equal logits) or whose cut
-// lies in the open last bin.
+// lies in the open last bin; it lists a bucket's members as soon as they fit,
+// as it does the boundary bin's of a top-k set that is longer than the list.
 //
 // Scratch of one (request, row): C * kRowArea bytes of
 //   Moments [C]              per-chunk sums behind the bin width
@@ -346,8 +347,9 @@ struct RowCut {
     float scale;  // (collect -> cut) wave_bin_scale of the row
 };
 // The candidates decide; nothing is cut; scan the row; the candidates decide
-// but have no room in the row's area; top-k keeps every valid logit.
-enum { kCutFound = 0, kCutAll = 1, kCutRow = 2, kCutGather = 3, kCutNoTopK = 4 };
+// but have no room in the row's area; top-k keeps every valid logit; the
+// boundary bin decides top-k's cut (the bins above it are too long a list).
+enum { kCutFound = 0, kCutAll = 1, kCutRow = 2, kCutGather = 3, kCutNoTopK = 4, kCutBin = 5 };
 
 // A row's record lies at the end of its area.
 __device__ __forceinline__ RowCut &row_cut(uint8_t *area, const Geo &g, int b, int row) {
@@ -568,7 +570,8 @@ __global__ __launch_bounds__(256) void accept_collect_kernel(const float *__rest
     int status = kCutFound;
     if (COUNT) {
         if (tot <= (T)top_k) status = kCutNoTopK;
-        else if (bnd >= tg.NB - 1 || upto_s > (T)tg.cap) status = kCutRow;
+        else if (bnd >= tg.NB - 1) status = kCutRow;
+        else if (upto_s > (T)tg.cap) status = upto_s - before_s <= (T)(tg.cap / 4 * 3) ? kCutBin : kCutRow;
         else if (upto_s > (T)(tg.KC * 4 * tg.seg)) status = kCutGather;
     } else {
         if (!(total > 0.0) || isinf(total) || bnd >= tg.NB) status = kCutAll;
@@ -637,6 +640,7 @@ struct SelShared {
     double total_w;     // all weight of the first pass
     uint32_t total_c;
     int id;             // result of an id selection
+    uint32_t seg_n[W];  // gather: members of each wave
     ExpEntry tab[16];
 };
 
@@ -845,17 +849,93 @@ __device__ int select_id(const float *p, int V, SelShared<W> &s, uint32_t key, C
     return id;
 }
 
+// The row's elements that `take` admits side by side in the list, by one
+// workgroup: each wave fills a segment in (iteration, lane) order, then the
+// segments close up. Returns their number, or -1 if a segment is too short.
+// Waves take every W-th 64 ids, so a run of large logits spreads over them.
+template <int W, class Take>
+__device__ __forceinline__ int gather(const float *__restrict__ p, int V, Member *list, uint32_t *found_s, Take take) {
+    constexpr int kT = 64 * W, kSeg = cand_most(W) / W, kPer = cand_most(W) / kT, kU = 8;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    uint32_t found = 0u;
+    for (int j0 = threadIdx.x; j0 - (int)threadIdx.x < V && found <= (uint32_t)kSeg; j0 += kU * kT) {
+        float l[kU];
+#pragma unroll
+        for (int u = 0; u < kU; u++) l[u] = j0 + kT * u < V ? p[j0 + kT * u] : NAN;
+#pragma unroll
+        for (int u = 0; u < kU; u++) {
+            const bool in = valid_logit(l[u]) && take(l[u]);
+            const uint64_t m = __ballot(in);
+            const uint32_t at = found + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+            if (in && at < (uint32_t)kSeg) list[wave * kSeg + at] = Member{l[u], j0 + kT * u};
+            found += (uint32_t)__popcll(m);
+        }
+    }
+    if (lane == 0) found_s[wave] = found;
+    __syncthreads();
+    uint32_t at[W + 1];
+    at[0] = 0u;
+    bool ok = true;
+#pragma unroll
+    for (int q = 0; q < W; q++) {
+        ok = ok && found_s[q] <= (uint32_t)kSeg;
+        at[q + 1] = at[q] + found_s[q];
+    }
+    const int n = (int)at[W];
+    Member m[kPer];
+#pragma unroll
+    for (int u = 0; u < kPer; u++) {
+        const uint32_t i = threadIdx.x + u * kT;
+        if (!ok || i >= (uint32_t)n) continue;
+        uint32_t from = 0u;
+#pragma unroll
+        for (int q = 0; q < W; q++)
+            if (i >= at[q]) from = q * kSeg + i - at[q];
+        m[u] = list[from];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kPer; u++) {
+        const uint32_t i = threadIdx.x + u * kT;
+        if (ok && i < (uint32_t)n) list[i] = m[u];
+    }
+    __syncthreads();
+    return ok ? n : -1;
+}
+
 // The cut of one row by radix selection over src. With `tail` (candidates of
 // one bin): the weight `before` lies ahead of src's elements, of `total`.
+// `room` (src is the whole row): a list of cand_most(W) for the members of
+// the chosen bucket once they are few enough, so that the later passes need
+// not read the row (8 x 2 x 127606, top-k 31901 of rows with one logit of 1e4:
+// 315 -> 286 us).
+// `bin_n` of them may be there already, those of the bin with top-k's cut,
+// behind `bin_before` larger ones (16 rows of 53144, top-k 13286: 103 -> 73 us;
+// 37 of 63461, top-k 15865, top-p 0.95: 222 -> 180).
 template <int W>
 __device__ __forceinline__ Cut radix_cut(const SelSrc src, SelShared<W> &s, float mx, const Temp t, int top_k, float top_p,
-                                         bool tail, double before, double total) {
+                                         bool tail, double before, double total, Member *room, int bin_n,
+                                         uint32_t bin_before) {
     Cut cut{0u, INT_MAX};
+    // (three quarters of the list: the waves' segments fill unevenly)
+    auto narrow = [&](SelSrc &cur, uint32_t mask, uint32_t pre) __attribute__((always_inline)) {
+        if (!room || cur.list || s.tc[s.bucket] > (uint32_t)(cand_most(W) / 4 * 3)) return;  // uniform
+        const int n = gather<W>(src.p, src.V, room, s.seg_n, [=](float l) { return (order_key(l) & mask) == pre; });
+        if (n < 0) return;
+        cur.list = room;
+        cur.n = n;
+    };
     // top-k: the top_k-th element in (logit desc, id asc) order (sampling.go:90-92).
     if (top_k > 0) {
+        SelSrc cur = src;
+        if (bin_n > 0) {
+            cur.list = room;
+            cur.n = bin_n;
+            cur.top = true;
+        }
         if (threadIdx.x == 0) {
             s.prefix = 0u;
-            s.before_c = 0u;
+            s.before_c = bin_n > 0 ? bin_before : 0u;
             s.before_w = 0.0;
         }
         __syncthreads();
@@ -864,7 +944,8 @@ __device__ __forceinline__ Cut radix_cut(const SelSrc src, SelShared<W> &s, floa
             const int shift = 24 - 8 * pass;
             const uint32_t mask = pass ? ~0u << (shift + 8) : 0u;
             const uint32_t pre = s.prefix;
-            hist_pass<false>(src, mx, t, s, shift, [=](uint32_t k, int) { return (k & mask) == pre; });
+            if (pass) narrow(cur, mask, pre);
+            hist_pass<false>(cur, mx, t, s, shift, [=](uint32_t k, int) { return (k & mask) == pre; });
             if (threadIdx.x < 64) {
                 uint32_t tot_c = s.total_c;
                 if (pass == 0) {
@@ -872,10 +953,10 @@ __device__ __forceinline__ Cut radix_cut(const SelSrc src, SelShared<W> &s, floa
                     bucket_totals(s, &tot_c, &unused);
                     if (threadIdx.x == 0) s.total_c = tot_c;
                 }
-                if (src.top || tot_c > (uint32_t)top_k) scan_buckets(s, true, false, (uint32_t)top_k, 0.0, shift);
+                if (cur.top || tot_c > (uint32_t)top_k) scan_buckets(s, true, false, (uint32_t)top_k, 0.0, shift);
             }
             __syncthreads();
-            if (!src.top && s.total_c <= (uint32_t)top_k) {
+            if (!cur.top && s.total_c <= (uint32_t)top_k) {
                 all = true;
                 break;
             }
@@ -900,13 +981,15 @@ __device__ __forceinline__ Cut radix_cut(const SelSrc src, SelShared<W> &s, floa
             s.before_w = tail ? before : 0.0;
         }
         __syncthreads();
+        SelSrc cur = src;
         bool found = true;
         for (int pass = 0; pass < 4 && found; pass++) {
             const int shift = 24 - 8 * pass;
             const uint32_t mask = pass ? ~0u << (shift + 8) : 0u;
             const uint32_t pre = s.prefix;
             const Cut ck = cut;
-            hist_pass<true>(src, mx, t, s, shift,
+            if (pass) narrow(cur, mask, pre);
+            hist_pass<true>(cur, mx, t, s, shift,
                             [=](uint32_t k, int j) { return in_cut(k, j, ck) && (k & mask) == pre; });
             if (threadIdx.x < 64) {
                 double tot = s.total_w;
@@ -953,63 +1036,6 @@ __device__ __forceinline__ double block_sum(double v, double *waves) {
     double t = 0.0;
     for (int w = 0; w < W; w++) t += waves[w];
     return t;
-}
-
-// A row's candidates (see accept_collect_kernel) side by side in the list, by
-// one workgroup: each wave fills a segment in (iteration, lane) order, then
-// the segments close up. Returns their number, or -1 if a segment is too
-// short. Waves take every sixteenth 64 ids, so a run of large logits spreads
-// over them.
-template <int W>
-__device__ __forceinline__ int gather(const float *__restrict__ p, int V, const RowCut &in, int NB, bool above,
-                                      Member *list, uint32_t *found_s) {
-    constexpr int kT = 64 * W, kSeg = cand_most(W) / W, kPer = cand_most(W) / kT, kU = 8;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    uint32_t found = 0u;
-    for (int j0 = threadIdx.x; j0 - (int)threadIdx.x < V && found <= (uint32_t)kSeg; j0 += kU * kT) {
-        float l[kU];
-#pragma unroll
-        for (int u = 0; u < kU; u++) l[u] = j0 + kT * u < V ? p[j0 + kT * u] : NAN;
-#pragma unroll
-        for (int u = 0; u < kU; u++) {
-            const int bin = bin_of(l[u], in.best_v, in.scale, NB);
-            const bool take = valid_logit(l[u]) && (above ? bin <= in.bnd : bin == in.bnd);
-            const uint64_t m = __ballot(take);
-            const uint32_t at = found + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-            if (take && at < (uint32_t)kSeg) list[wave * kSeg + at] = Member{l[u], j0 + kT * u};
-            found += (uint32_t)__popcll(m);
-        }
-    }
-    if (lane == 0) found_s[wave] = found;
-    __syncthreads();
-    uint32_t at[W + 1];
-    at[0] = 0u;
-    bool ok = true;
-#pragma unroll
-    for (int q = 0; q < W; q++) {
-        ok = ok && found_s[q] <= (uint32_t)kSeg;
-        at[q + 1] = at[q] + found_s[q];
-    }
-    const int n = (int)at[W];
-    Member m[kPer];
-#pragma unroll
-    for (int u = 0; u < kPer; u++) {
-        const uint32_t i = threadIdx.x + u * kT;
-        if (!ok || i >= (uint32_t)n) continue;
-        uint32_t from = 0u;
-#pragma unroll
-        for (int q = 0; q < W; q++)
-            if (i >= at[q]) from = q * kSeg + i - at[q];
-        m[u] = list[from];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < kPer; u++) {
-        const uint32_t i = threadIdx.x + u * kT;
-        if (ok && i < (uint32_t)n) list[i] = m[u];
-    }
-    __syncthreads();
-    return ok ? n : -1;
 }
 
 // One workgroup per row: the exact cut, and the kept weight without the
@@ -1095,7 +1121,10 @@ __global__ __launch_bounds__(64 * W, 4) void accept_cut_kernel(const float *__re
     }
     int n = fits ? n_s : 0;
     if (!fits && (in.status == kCutFound || in.status == kCutGather)) {
-        n = gather<W>(p, g.V, in, tg.NB, top_k > 0, list, seg_at);
+        n = gather<W>(p, g.V, list, s.seg_n, [=](float l) {
+            const int bin = bin_of(l, in.best_v, in.scale, tg.NB);
+            return top_k > 0 ? bin <= in.bnd : bin == in.bnd;
+        });
         fits = n >= 0;
     }
     Cut cut{0u, INT_MAX};
@@ -1160,7 +1189,12 @@ __global__ __launch_bounds__(64 * W, 4) void accept_cut_kernel(const float *__re
         cut = Cut{(uint32_t)(last >> 32), (int32_t)~(uint32_t)last};
     } else {
         const SelSrc src{p, g.V, fits || direct == 1 ? list : nullptr, fits ? n : g.V, fits && top_k > 0};
-        cut = radix_cut(src, s, mx, t, in.status == kCutNoTopK ? 0 : top_k, top_p, fits && top_k <= 0, in.before, in.total);
+        int bin_n = 0;
+        if (in.status == kCutBin)
+            bin_n = gather<W>(p, g.V, list, s.seg_n,
+                              [=](float l) { return bin_of(l, in.best_v, in.scale, tg.NB) == in.bnd; });
+        cut = radix_cut(src, s, mx, t, in.status == kCutNoTopK ? 0 : top_k, top_p, fits && top_k <= 0, in.before, in.total,
+                        direct ? nullptr : list, bin_n, (uint32_t)in.before);
         __syncthreads();
     }
     // the kept weight: candidates (after the bins above them), or the row

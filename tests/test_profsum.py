@@ -1,9 +1,11 @@
 """yuuka_amd.profsum: per-kernel summary of a rocprofv3 CSV directory,
 restricted to the last N verify steps (each ends with one
-accept_finalize_kernel)."""
+accept_finalize_kernel, or accept_pick_kernel)."""
 from __future__ import annotations
 
 import csv
+
+import pytest
 
 from yuuka_amd import profsum
 
@@ -21,14 +23,15 @@ def _trace(tmp_path, names):
     return str(tmp_path)
 
 
-def test_steps_window_and_names(tmp_path):
-    fin = "void yk::(anonymous namespace)::accept_finalize_kernel<true>(yk::Args)"
+@pytest.mark.parametrize("last", ["accept_finalize_kernel", "accept_pick_kernel"])
+def test_steps_window_and_names(tmp_path, last):
+    fin = f"void yk::(anonymous namespace)::{last}<true>(yk::Args)"
     gemm = "void yk::fgemm_stream_kernel<12, 2, 4, 0, true>(yk::FusedGemmArgs)"
     seq = [(gemm, 99000), (fin, 1000)]            # warm-up step: outside the window
     seq += [(gemm, 10000), (gemm, 20000), (fin, 2000)] * 2
     out = profsum.summarise(profsum.load(_trace(tmp_path, seq)), steps=1)
     rows = {r.split("|")[1].strip(): r.split("|")[2:5] for r in out.splitlines() if r.startswith("| `")}
-    assert set(rows) == {"`fgemm_stream_kernel`", "`accept_finalize_kernel`"}
+    assert set(rows) == {"`fgemm_stream_kernel`", f"`{last}`"}
     n, avg, per_step = (x.strip() for x in rows["`fgemm_stream_kernel`"])
     assert (n, avg, per_step) == ("2", "15.00", "30.0")
     assert out.splitlines()[-1].startswith("| total | 3 | | 32.0 |")

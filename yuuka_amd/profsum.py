@@ -4,8 +4,9 @@
     python3 -m yuuka_amd.profsum DIR [--steps N] [--by-grid] [--templates] [--counters]
 
 ``--steps N`` keeps the dispatches of the last N verify steps: those after
-the (N+1)-th-from-last ``accept_finalize_kernel`` up to the last one (every
-verify step ends with exactly one). Kernel names are shown without namespace
+the (N+1)-th-from-last ``accept_finalize_kernel`` (with top-k / top-p:
+``accept_pick_kernel``) up to the last one (every verify step ends with exactly
+one). Kernel names are shown without namespace
 or template arguments; ``--by-grid`` splits a kernel's rows by grid size and
 ``--templates`` by template arguments.
 With ``--counters`` the per-dispatch average of every collected counter is
@@ -52,7 +53,7 @@ def summarise(disp: dict, steps: int = 0, by_grid: bool = False, counters: bool 
               templates: bool = False) -> str:
     ids = sorted(disp)
     if steps:
-        acc = [i for i in ids if base_name(disp[i]["name"]) == "accept_finalize_kernel"]
+        acc = [i for i in ids if base_name(disp[i]["name"]) in ("accept_finalize_kernel", "accept_pick_kernel")]
         if len(acc) < steps + 1:
             raise SystemExit(f"only {len(acc)} verify steps in the trace, {steps + 1} needed")
         first = acc[-(steps + 1)]

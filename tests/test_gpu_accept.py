@@ -226,7 +226,8 @@ def test_truncation_tie_group_spanning_late_id_steps(dev, stream):
 # (equal logits fill one bin) or the cut is in the open last bin. A sorted row
 # fills one wave's segment; a masked row may have fewer valid logits than top-k.
 # More than 8192 of top-k are cut among the boundary bin's members, and a
-# selection over the row lists a bucket's members once they are few enough.
+# selection over the row lists a bucket's members once they are few enough. With
+# top-k the first bin takes logits far above the others.
 @pytest.mark.parametrize("V,shape,top_k,top_p,T", [
     (8192, "normal", 0, 0.9, 0.7), (8193, "normal", 0, 0.9, 0.7), (8193, "normal", 513, 0.97, 1.0),
     (40001, "narrow", 0, 0.6, 1.0), (40001, "normal", 511, 1.0, 0.8), (40001, "normal", 6000, 0.999, 1.3),
@@ -238,7 +239,9 @@ def test_truncation_tie_group_spanning_late_id_steps(dev, stream):
     (16385, "normal", 40, 1.0, 0.7), (12000, "masked", 5000, 1.0, 1.0), (40001, "masked", 6000, 1.0, 0.7),
     (40001, "masked", 6000, 0.8, 0.7), (40001, "normal", 9000, 1.0, 1.0), (40001, "normal", 20000, 0.9, 1.3),
     (40001, "coarse", 9001, 1.0, 1.0), (40001, "coarse", 9001, 0.95, 1.3), (40001, "coarse", 0, 0.97, 1.3),
-    (40001, "outlier", 200, 1.0, 1.0), (40001, "outlier", 9000, 0.9, 5e3), (40001, "outlier", 0, 0.99, 5e3)])
+    (40001, "outlier", 200, 1.0, 1.0), (40001, "outlier", 9000, 0.9, 5e3), (40001, "outlier", 0, 0.99, 5e3),
+    (40001, "heads", 40, 1.0, 1e3), (40001, "heads", 40, 0.5, 1e3), (40001, "heads", 600, 0.999, 1e3),
+    (40001, "lowest", 50, 0.9, 1.0), (40001, "lowest", 9000, 1.0, 1.0)])
 def test_truncation_paths_match_oracle(dev, stream, V, shape, top_k, top_p, T):
     rng = np.random.default_rng(V + top_k)
     k = 3
@@ -255,6 +258,10 @@ def test_truncation_paths_match_oracle(dev, stream, V, shape, top_k, top_p, T):
         logits[rng.random(logits.shape) < 0.98] = -np.inf
     if shape == "outlier":
         logits[:, V // 2] = -1e30
+    if shape == "heads":  # fifty logits far above the others, a few of them tied
+        logits[:, 100:5100:100] = 1e4 + rng.integers(0, 40, (k + 1, 50))
+    if shape == "lowest":
+        logits[rng.random(logits.shape) < 0.98] = np.finfo(np.float32).min
     drafts = np.argsort(-logits, axis=1, kind="stable")[np.arange(k), [0, 1, 5]].astype(np.int32)
     for step in range(3):
         assert _check_truncated(dev, stream, logits, drafts, T, top_k, top_p, 19, step) == 0

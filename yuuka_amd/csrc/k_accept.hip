@@ -332,6 +332,11 @@ struct TruncGeo {
     uint32_t bins_off, cnt_off, cand_off;  // in the row's area
 };
 
+// See wave_bin_map.
+struct BinMap {
+    float top, scale;
+};
+
 // What collect leaves for a row.
 struct RowCut {
     Cut cut;
@@ -344,7 +349,7 @@ struct RowCut {
     int best_i;
     int status;
     int bnd;      // (collect -> cut) the boundary bin
-    float scale;  // (collect -> cut) wave_bin_scale of the row
+    BinMap map;   // (collect -> cut) the row's bins
 };
 // The candidates decide; nothing is cut; scan the row; the candidates decide
 // but have no room in the row's area; top-k keeps every valid logit; the
@@ -356,13 +361,17 @@ __device__ __forceinline__ RowCut &row_cut(uint8_t *area, const Geo &g, int b, i
     return *reinterpret_cast<RowCut *>(row_area(area, g, b, row) + g.C * kRowArea - sizeof(RowCut));
 }
 
-// Bins per unit of logit below the maximum: the range down to three standard
-// deviations under the mean in NB steps; weighed bins (COUNT false) end at
-// 48 T if that is less (the weights below it are under 1e-20 of the largest).
-// Every workgroup of a row computes the same value (fixed order), so the bins
-// of its passes agree. Wave 0 of a workgroup.
+// The bins of a row: `scale` of them per unit of logit below `top`, over the
+// range down to three standard deviations under the mean in NB steps. Weighed
+// bins (COUNT false) start at the maximum and end at 48 T if that is less (the
+// weights below it are under 1e-20 of the largest); counted ones start at most
+// eight deviations above the mean, or one logit far above the others would
+// leave these a few bins (13 x 9 x 127103, top-k 5000, one logit of 1e4:
+// 383 -> 134 us).
+// Every workgroup of a row computes the same values (fixed order, every fused
+// operation written out), so the bins of its passes agree. Wave 0 of a workgroup.
 template <bool COUNT>
-__device__ __forceinline__ float wave_bin_scale(const Moments *__restrict__ m, int C, float mx, const Temp &t, int NB) {
+__device__ __forceinline__ BinMap wave_bin_map(const Moments *__restrict__ m, int C, float mx, const Temp &t, int NB) {
     const int lane = threadIdx.x & 63;
     float n = 0.f, s1 = 0.f, s2 = 0.f;
     for (int c = lane; c < C; c += 64) {
@@ -377,16 +386,18 @@ __device__ __forceinline__ float wave_bin_scale(const Moments *__restrict__ m, i
     }
     const float cap = fminf(fmaxf(48.f * (float)t.t, 1e-30f), 1e30f);
     const float mean = s1 / n;
-    const float sd = sqrtf(fmaxf(s2 / n - mean * mean, 1e-6f * mean * mean));
-    float range = (mx - mean) + 3.f * sd;
+    const float sd = sqrtf(fmaxf(fmaf(-mean, mean, s2 / n), 1e-6f * mean * mean));
+    const float top = COUNT ? fminf(mx, fmaf(8.f, sd, mean)) : mx;  // (mx if n is 0)
+    float range = fmaf(3.f, sd, top - mean);
     if (!(range > 1e-30f && range < (COUNT ? 1e30f : cap))) range = cap;
-    return (float)NB / range;
+    return BinMap{top, (float)NB / range};
 }
 
 // Monotone: a larger logit never has a larger bin (each operation rounds
-// monotonically; the last bin is open, and takes a NaN).
-__device__ __forceinline__ int bin_of(float l, float mx, float scale, int NB) {
-    return (int)fminf((mx - l) * scale, (float)(NB - 1));
+// monotonically; the first bin takes what is above `top`, the last one is
+// open, and takes a NaN).
+__device__ __forceinline__ int bin_of(float l, const BinMap &m, int NB) {
+    return (int)fmaxf(fminf((m.top - l) * m.scale, (float)(NB - 1)), 0.f);
 }
 
 // Histogram of one chunk of a row, the draft's weight left out. COUNT (with
@@ -401,7 +412,8 @@ __global__ __launch_bounds__(64 * kBinWaves) void accept_bins_kernel(const float
     using T = typename std::conditional<COUNT, uint32_t, double>::type;
     extern __shared__ __attribute__((aligned(16))) uint8_t bins_dyn[];
     T *hist = reinterpret_cast<T *>(bins_dyn);  // [wave][NB]
-    __shared__ float mx_s, scale_s;
+    __shared__ float mx_s;
+    __shared__ BinMap map_s;
     __shared__ ExpEntry tab[16];
     const ExpEntry entry = exp_entry();
     constexpr int kT = 64 * kBinWaves;
@@ -417,15 +429,16 @@ __global__ __launch_bounds__(64 * kBinWaves) void accept_bins_kernel(const float
     for (int i = threadIdx.x; i < kBinWaves * tg.NB; i += kT) hist[i] = (T)0;
     if (threadIdx.x < 64) {
         const Stat s = wave_best(stats + ((uint64_t)b * g.R + row) * g.C, g.C);
-        const float sc = wave_bin_scale<COUNT>(reinterpret_cast<const Moments *>(ra), g.C, s.v, t, tg.NB);
+        const BinMap map = wave_bin_map<COUNT>(reinterpret_cast<const Moments *>(ra), g.C, s.v, t, tg.NB);
         if (threadIdx.x == 0) {
             mx_s = s.v;
-            scale_s = sc;
+            map_s = map;
         }
     }
     put_exp_entry(tab, entry);
     __syncthreads();
-    const float mx = mx_s, scale = scale_s;
+    const float mx = mx_s;
+    const BinMap map = map_s;
     const int d = !COUNT && row < g.k ? drafts[(uint64_t)b * g.ds + row] : -1;
     T *mine = hist + (threadIdx.x >> 6) * tg.NB;
     while (j0 < end) {
@@ -436,7 +449,7 @@ __global__ __launch_bounds__(64 * kBinWaves) void accept_bins_kernel(const float
         if constexpr (COUNT) {
 #pragma unroll
             for (int u = 0; u < kU; u++)
-                if (valid_logit(lv[u])) atomicAdd(&mine[bin_of(lv[u], mx, scale, tg.NB)], 1u);
+                if (valid_logit(lv[u])) atomicAdd(&mine[bin_of(lv[u], map, tg.NB)], 1u);
         } else {
             // four weights at a time without branches: their chains of
             // dependent float64 operations interleave
@@ -450,7 +463,7 @@ __global__ __launch_bounds__(64 * kBinWaves) void accept_bins_kernel(const float
                 for (int u = 0; u < kW; u++) {
                     const float l = lv[u0 + u];
                     if (valid_logit(l) && j0 + kT * (u0 + u) != d)
-                        unsafeAtomicAdd(&mine[bin_of(l, mx, scale, tg.NB)], w[u]);
+                        unsafeAtomicAdd(&mine[bin_of(l, map, tg.NB)], w[u]);
                 }
             }
         }
@@ -479,7 +492,8 @@ __global__ __launch_bounds__(256) void accept_collect_kernel(const float *__rest
                                                              const Stat *__restrict__ stats, int top_k, float top_p,
                                                              Temp t, uint8_t *__restrict__ area) {
     using T = typename std::conditional<COUNT, uint32_t, double>::type;
-    __shared__ float mx_s, scale_s;
+    __shared__ float mx_s;
+    __shared__ BinMap map_s;
     __shared__ int best_i_s, bnd_s;
     __shared__ T wave_tot[4];
     __shared__ T before_s, upto_s;
@@ -502,10 +516,10 @@ __global__ __launch_bounds__(256) void accept_collect_kernel(const float *__rest
             if (i < per && lo + i < tg.NB) h[i] += hist[(uint64_t)ch * tg.NB + lo + i];
     if (threadIdx.x < 64) {
         const Stat s = wave_best(stats + ((uint64_t)b * g.R + row) * g.C, g.C);
-        const float sc = wave_bin_scale<COUNT>(reinterpret_cast<const Moments *>(ra), g.C, s.v, t, tg.NB);
+        const BinMap map = wave_bin_map<COUNT>(reinterpret_cast<const Moments *>(ra), g.C, s.v, t, tg.NB);
         if (threadIdx.x == 0) {
             mx_s = s.v;
-            scale_s = sc;
+            map_s = map;
             best_i_s = s.i;
             bnd_s = tg.NB;
             before_s = upto_s = (T)0;
@@ -525,7 +539,8 @@ __global__ __launch_bounds__(256) void accept_collect_kernel(const float *__rest
     if (lane == 63) wave_tot[wave] = inc;
     put_exp_entry(tab, entry);
     __syncthreads();
-    const float mx = mx_s, scale = scale_s;
+    const float mx = mx_s;
+    const BinMap map = map_s;
     T tot = (T)0;
     for (int w = 0; w < 4; w++) {
         if (w == wave) exc += tot;
@@ -537,7 +552,7 @@ __global__ __launch_bounds__(256) void accept_collect_kernel(const float *__rest
     int dbin = tg.NB;
     if (!COUNT && d >= 0 && d < g.V && valid_logit(p[d])) {
         wd = soft_weight(p[d], mx, t, tab);
-        dbin = bin_of(p[d], mx, scale, tg.NB);
+        dbin = bin_of(p[d], map, tg.NB);
     }
     const double total = (double)tot + wd;
     {
@@ -589,7 +604,7 @@ __global__ __launch_bounds__(256) void accept_collect_kernel(const float *__rest
         o.best_i = best_i_s;
         o.status = status;
         o.bnd = bnd;
-        o.scale = scale;
+        o.map = map;
     }
     const int w = c * 4 + wave;
     uint32_t found = 0u;
@@ -603,7 +618,7 @@ __global__ __launch_bounds__(256) void accept_collect_kernel(const float *__rest
             for (int u = 0; u < kU; u++) l[u] = j0 + 256 * u < end ? p[j0 + 256 * u] : NAN;
 #pragma unroll
             for (int u = 0; u < kU; u++) {
-                const int bin = bin_of(l[u], mx, scale, tg.NB);
+                const int bin = bin_of(l[u], map, tg.NB);
                 const bool take = valid_logit(l[u]) && (COUNT ? bin <= bnd : bin == bnd);
                 const uint64_t m = __ballot(take);
                 if (!m) continue;
@@ -907,11 +922,10 @@ __device__ __forceinline__ int gather(const float *__restrict__ p, int V, Member
 // one bin): the weight `before` lies ahead of src's elements, of `total`.
 // `room` (src is the whole row): a list of cand_most(W) for the members of
 // the chosen bucket once they are few enough, so that the later passes need
-// not read the row (8 x 2 x 127606, top-k 31901 of rows with one logit of 1e4:
-// 315 -> 286 us).
-// `bin_n` of them may be there already, those of the bin with top-k's cut,
-// behind `bin_before` larger ones (16 rows of 53144, top-k 13286: 103 -> 73 us;
-// 37 of 63461, top-k 15865, top-p 0.95: 222 -> 180).
+// not read the row. `bin_n` of them may be there already, those of the bin
+// with top-k's cut, behind `bin_before` larger ones (16 rows of 53144, top-k
+// 13286: 103 -> 73 us; with a bucket's list for top-p, 37 rows of 63461, top-k
+// 15865, top-p 0.95: 222 -> 180).
 template <int W>
 __device__ __forceinline__ Cut radix_cut(const SelSrc src, SelShared<W> &s, float mx, const Temp t, int top_k, float top_p,
                                          bool tail, double before, double total, Member *room, int bin_n,
@@ -1122,7 +1136,7 @@ __global__ __launch_bounds__(64 * W, 4) void accept_cut_kernel(const float *__re
     int n = fits ? n_s : 0;
     if (!fits && (in.status == kCutFound || in.status == kCutGather)) {
         n = gather<W>(p, g.V, list, s.seg_n, [=](float l) {
-            const int bin = bin_of(l, in.best_v, in.scale, tg.NB);
+            const int bin = bin_of(l, in.map, tg.NB);
             return top_k > 0 ? bin <= in.bnd : bin == in.bnd;
         });
         fits = n >= 0;
@@ -1192,7 +1206,7 @@ __global__ __launch_bounds__(64 * W, 4) void accept_cut_kernel(const float *__re
         int bin_n = 0;
         if (in.status == kCutBin)
             bin_n = gather<W>(p, g.V, list, s.seg_n,
-                              [=](float l) { return bin_of(l, in.best_v, in.scale, tg.NB) == in.bnd; });
+                              [=](float l) { return bin_of(l, in.map, tg.NB) == in.bnd; });
         cut = radix_cut(src, s, mx, t, in.status == kCutNoTopK ? 0 : top_k, top_p, fits && top_k <= 0, in.before, in.total,
                         direct ? nullptr : list, bin_n, (uint32_t)in.before);
         __syncthreads();

@@ -462,7 +462,7 @@ __global__ __launch_bounds__(64 * kBinWaves) void accept_bins_kernel(const float
 #pragma unroll
                 for (int u = 0; u < kW; u++) {
                     const float l = lv[u0 + u];
-                    if (valid_logit(l) && j0 + kT * (u0 + u) != d)
+                    if (valid_logit(l) && w[u] != 0.0 && j0 + kT * (u0 + u) != d)
                         unsafeAtomicAdd(&mine[bin_of(l, map, tg.NB)], w[u]);
                 }
             }

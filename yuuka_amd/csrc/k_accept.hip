@@ -1056,8 +1056,8 @@ __device__ __forceinline__ double block_sum(double v, double *waves) {
 // draft and of the draft. Up to kRankMost candidates are put in order by
 // counting (thread i counts what lies ahead of candidate i) and their weights
 // summed in that order (some 450 candidates of one row: 63 us a call; with the
-// sums taken in the counting loop 82); more take the radix selection. `direct`: no candidates were collected, the row itself is
-// taken (1: into LDS).
+// sums taken in the counting loop 82); more take the radix selection.
+// `direct`: no candidates were collected, the row itself is taken (1: into LDS).
 template <int W>
 __global__ __launch_bounds__(64 * W, 4) void accept_cut_kernel(const float *__restrict__ logits, Geo g, TruncGeo tg,
                                                                     const int32_t *__restrict__ drafts,
@@ -1692,9 +1692,10 @@ int cut_waves(int rows) { return rows <= 256 ? 16 : 8; }
 
 // The layout of a row's area. A chunk has a few thousand logits, or the
 // workgroups do little but add up the histograms (20 rows of 8200..32000,
-// top-p 0.9, with up to 52 chunks of a row: 56 us; now 39..43). The bins take at most about half of it, the
-// candidates the rest; few rows have many chunks and much room, thousands of
-// rows little (fewer bins, and more of their rows scan the row).
+// top-p 0.9, with up to 52 chunks of a row: 56 us; now 39..43). The bins take
+// at most about half of it, the candidates the rest; few rows have many chunks
+// and much room, thousands of rows little (fewer bins, and more of their rows'
+// candidates are gathered by the cut's workgroup).
 TruncGeo trunc_geo(const Geo &g) {
     TruncGeo t;
     const int rows = g.B * g.R;
@@ -1777,7 +1778,9 @@ hipError_t launch_verify_accept(const float *logits, const int32_t *drafts, int3
         attr = true;
     }
     int cand = tg.cap;
-    const int direct = (int)p.vocab <= kDirectMost ? (g.V <= tg.cap ? 1 : 2) : (top_k_on && !top_p_on && g.V <= kDirectTopK && g.B * g.R <= 256 ? 2 : 0);
+    int direct = 0;
+    if (g.V <= kDirectMost) direct = g.V <= tg.cap ? 1 : 2;
+    else if (top_k_on && !top_p_on && g.V <= kDirectTopK && g.B * g.R <= 256) direct = 2;
     if (direct) {
         accept_stats_kernel<false><<<sgrid, 256, 0, stream>>>(logits, g, stats, vec, wpc, nullptr);
         cand = direct == 1 ? g.V : 0;

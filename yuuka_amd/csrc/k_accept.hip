@@ -1767,16 +1767,16 @@ hipError_t launch_verify_accept(const float *logits, const int32_t *drafts, int3
     const dim3 rgrid((unsigned)g.R, (unsigned)g.B);
     const dim3 hgrid((unsigned)tg.HC, (unsigned)g.R, (unsigned)g.B), kgrid((unsigned)tg.KC, (unsigned)g.R, (unsigned)g.B);
     const uint32_t bins_lds = (uint32_t)(kBinWaves * tg.NB) * (top_k_on ? 4u : 8u);
-    static bool attr = false;
-    if (!attr) {
+    static const bool attr = [] {  // (once, also with several threads)
         (void)hipFuncSetAttribute(reinterpret_cast<const void *>(accept_cut_kernel<16>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, cand_most(16) * (int)sizeof(Member));
         (void)hipFuncSetAttribute(reinterpret_cast<const void *>(accept_cut_kernel<8>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, cand_most(8) * (int)sizeof(Member));
         (void)hipFuncSetAttribute(reinterpret_cast<const void *>(accept_bins_kernel<false>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, kBinWaves * kBins * 8);
-        attr = true;
-    }
+        return true;
+    }();
+    (void)attr;
     int cand = tg.cap;
     int direct = 0;
     if (g.V <= kDirectMost) direct = g.V <= tg.cap ? 1 : 2;
